@@ -70,6 +70,74 @@ std::vector<FwdChunk> make_chunks(const std::vector<FwdAngle>& sorted, int nd, i
     return out;
 }
 
+// Tables of the sheared forward projection (FwdLine, FwdBin, Shear of
+// common.h) for class-sorted angles; false where the form does not apply.
+struct ShearTables {
+    std::vector<Shear> shear;
+    std::vector<FwdLine> lines;
+    std::vector<int> line0;
+    std::vector<FwdBin> bins;
+};
+
+bool make_shear(const std::vector<FwdAngle>& fa, int nd, int nlines, ShearTables& T)
+{
+    const int na = (int)fa.size();
+    // |mcand| <= 1: three bins per item; >= FWD_SHEAR_MIN: at most
+    // FWD_BIN_ITEMS items per bin, and not many more items than bins.  An
+    // offset beyond +-1e6 bins could overflow an item's line index.
+    for (const FwdAngle& A : fa) {
+        const double m = std::fabs((double)A.mcand);
+        if (!(m >= FWD_SHEAR_MIN && m <= 1.0 && std::fabs((double)A.off) < 1e6)) return false;
+    }
+    auto nearest = [](double x) { return (long long)(x + (x < 0 ? -0.5 : 0.5)); };
+    T.shear.reserve((size_t)na * nlines);
+    T.lines.reserve((size_t)na * (size_t)((nd + 4) / FWD_SHEAR_MIN));
+    T.bins.reserve((size_t)na * nd);
+    std::vector<int> m, cnt;
+    for (int a = 0; a < na; ++a) {
+        // products of these floats and a line's or candidate's number are exact
+        const double ms = fa[a].mstep, mc = fa[a].mcand, off = fa[a].off, inv = 1.0 / mc;
+        auto bin = [&](long long j) { return nearest((double)j * mc + off); };
+        // items whose nearest bin is -1 .. nd
+        long long j0 = (long long)std::floor(((mc > 0 ? -1.5 : nd + 0.5) - off) / mc) - 2;
+        auto in = [&](long long j) { return bin(j) >= -1 && bin(j) <= nd; };
+        while (!in(j0)) ++j0;
+        const size_t first = T.lines.size();
+        T.line0.push_back((int)first);
+        m.clear();
+        for (long long j = j0; in(j); ++j) {
+            m.push_back((int)bin(j));
+            T.lines.push_back(FwdLine{(int)j, (float)((double)j * mc + off - (double)m.back())});
+        }
+        const size_t b0 = T.bins.size();
+        T.bins.resize(b0 + nd, FwdBin{0, 0});
+        cnt.assign(nd, 0);
+        for (int i = 0; i < (int)m.size(); ++i)
+            for (int b = std::max(0, m[i] - 1); b <= std::min(nd - 1, m[i] + 1); ++b) {
+                FwdBin& B = T.bins[b0 + b];
+                if (cnt[b] == 0) B.first = i;
+                if (cnt[b] >= FWD_BIN_ITEMS || i != B.first + cnt[b]) return false;
+                B.code |= (b - m[i] + 2) << (3 * cnt[b]++);
+            }
+        for (int l = 0; l < nlines; ++l) {
+            const long long s = nearest(-l * ms * inv);
+            T.shear.push_back(Shear{(float)(l * ms + (double)s * mc), (int)s});
+        }
+    }
+    T.line0.push_back((int)T.lines.size());
+    return true;
+}
+
+template <typename T>
+int upload(const std::vector<T>& v, T** out)
+{
+    *out = nullptr;
+    if (v.empty()) return GR_OK;
+    GR_HIP(hipMalloc(out, sizeof(T) * v.size()));
+    GR_HIP(hipMemcpy(*out, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
+    return GR_OK;
+}
+
 hipStream_t stream_of(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
 bool valid_params(const gr_geometry* g, const gr_tgv_params* p)
@@ -139,6 +207,7 @@ ProbDev make_prob(const gr_geometry* gg, const gr_tgv_params* p, const gr_tgv_st
     P.fuse_primal = g.fuse_primal;
     P.ofs = reinterpret_cast<const float4*>(g.ofs_dev);
     P.fwd = g.fwd_dev;
+    set_shear(P, g);
     P.u = s->u; P.ubar = s->ubar; P.p = s->p; P.pbar = s->pbar; P.v = s->v; P.w = s->w;
     P.lam = s->lam; P.ktl = s->ktl; P.ku = s->ku; P.f = s->f; P.mfac = s->mfac;
     P.halo_ubar_hi = s->halo_ubar_hi; P.halo_pbar_lo = s->halo_pbar_lo;
@@ -233,7 +302,8 @@ int iterate_single(const gr_geometry* gg, const ProbDev& P, int n_iter, int ku_o
     for (int k = 0; k < 5; ++k) ms[k] = 0.0;
     Timer t(ms_out != nullptr, st);
     auto fwd_mode = [&](int it) {
-        return pmode | ((ku_on_last && it == n_iter - 1) ? FWD_WRITE : 0);
+        return pmode | (P.fuse_primal ? 0 : FWD_SCRATCH) |
+               ((ku_on_last && it == n_iter - 1) ? FWD_WRITE : 0);
     };
     const bool fused = s && s->u2 && s->v2 && (!P.tgv || s->w2) && !P.fuse_primal &&
                        n_iter >= 2;
@@ -303,11 +373,16 @@ struct gr_plan {
     int nprob = 0;
     std::vector<ProbDev> probs;
     ProbDev* probs_dev = nullptr;
-    struct FwdLaunch { int K, mi; size_t lds; std::vector<FwdItem> items; FwdItem* dev; };
+    // mi: items per thread, or 0: by lines, in work-groups of `waves` waves
+    struct FwdLaunch {
+        int K, mi; size_t lds; std::vector<FwdItem> items; FwdItem* dev; int waves = 0;
+    };
     struct AdjLaunch { int K, dim, tgv, fuse; size_t lds; std::vector<AdjItem> items; AdjItem* dev; };
     struct PrimalLaunch { int dim, tgv; std::vector<DualItem> items; DualItem* dev; };
     struct DualLaunch { int dim, coupling, tgv, maxc; std::vector<DualItem> items; DualItem* dev; };
     std::vector<FwdLaunch> fwd;
+    std::vector<DualItem> tiles;  // 32 x 32 tiles transposed ahead of the launches by lines
+    DualItem* tiles_dev = nullptr;
     std::vector<AdjLaunch> adj;
     std::vector<DualLaunch> dual;
     std::vector<PrimalLaunch> primal;
@@ -330,6 +405,8 @@ void plan_free_device(gr_plan* pl)
     if (pl->probs_dev) (void)hipFree(pl->probs_dev);
     pl->probs_dev = nullptr;
     for (auto& l : pl->fwd) if (l.dev) (void)hipFree(l.dev);
+    if (pl->tiles_dev) (void)hipFree(pl->tiles_dev);
+    pl->tiles_dev = nullptr;
     for (auto& l : pl->adj) if (l.dev) (void)hipFree(l.dev);
     for (auto& l : pl->dual) if (l.dev) (void)hipFree(l.dev);
     for (auto& l : pl->primal) if (l.dev) (void)hipFree(l.dev);
@@ -338,20 +415,11 @@ void plan_free_device(gr_plan* pl)
     pl->graph_block = 0;
 }
 
-template <typename T>
-int upload(const std::vector<T>& v, T** out)
-{
-    *out = nullptr;
-    if (v.empty()) return GR_OK;
-    GR_HIP(hipMalloc(out, sizeof(T) * v.size()));
-    GR_HIP(hipMemcpy(*out, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
-    return GR_OK;
-}
-
 int plan_build(gr_plan* pl, const gr_geometry* const* geoms)
 {
     plan_free_device(pl);
     pl->fwd.clear();
+    pl->tiles.clear();
     pl->adj.clear();
     pl->dual.clear();
     pl->primal.clear();
@@ -381,6 +449,11 @@ int plan_build(gr_plan* pl, const gr_geometry* const* geoms)
             }
         }
     }
+    // waves per work-group of the launches by lines
+    int line_waves = FWD_LINE_WAVES;
+    for (int i = 0; i < n; ++i)
+        if (fwd_by_lines(pl->probs[i], geoms[i]->g))
+            line_waves = std::max(line_waves, geoms[i]->g.shear_waves);
     std::map<std::tuple<int, int>, size_t> fwd_idx;
     std::map<std::tuple<int, int, int, int>, size_t> adj_idx;
     std::map<std::tuple<int, int>, size_t> primal_idx;
@@ -390,20 +463,40 @@ int plan_build(gr_plan* pl, const gr_geometry* const* geoms)
         const Geometry& g = geoms[i]->g;
         const int S = P.nz * P.nch;
         const int K = slice_group(S);
-        // forward items: slice groups x chunks (group-major)
-        const int t = tsel[i], mi = 8 >> t;
-        auto fk = std::make_tuple(K, mi);
-        if (!fwd_idx.count(fk)) {
-            fwd_idx[fk] = pl->fwd.size();
-            pl->fwd.push_back({K, mi, 0, {}, nullptr});
-        }
-        auto& fl = pl->fwd[fwd_idx[fk]];
-        fl.lds = std::max(fl.lds, fwd_lds_bytes(P, K));
-        for (int s0 = 0; s0 < S; s0 += K)
-            for (int c = g.tab_off[t]; c < g.tab_off[t + 1]; ++c) {
-                const FwdChunk& ch = g.chunks_host[c];
-                fl.items.push_back(FwdItem{i, ch.cls, ch.a0, ch.na, ch.b0, ch.nb, s0, 0});
+        if (fwd_by_lines(P, g)) {
+            // slice groups x runs of angles that fill line_waves waves of items
+            const int J = g.shear_waves;
+            auto fk = std::make_tuple(K, 0);
+            if (!fwd_idx.count(fk)) {
+                fwd_idx[fk] = pl->fwd.size();
+                pl->fwd.push_back({K, 0, 0, {}, nullptr});
+                pl->fwd.back().waves = line_waves;
             }
+            auto& fl = pl->fwd[fwd_idx[fk]];
+            const int per = line_waves / J;
+            for (int s0 = 0; s0 < S; s0 += K)
+                for (int a = 0; a < P.na; a += per)
+                    fl.items.push_back(FwdItem{i, J, a, std::min(per, P.na - a), 0, 0, s0, 0});
+            for (int sl = 0; sl < S; ++sl)
+                for (int y0 = 0; y0 < P.ny; y0 += 32)
+                    for (int x0 = 0; x0 < P.nx; x0 += 32)
+                        pl->tiles.push_back(DualItem{i, x0, y0, sl});
+        } else {
+            // slice groups x chunks (group-major)
+            const int t = tsel[i], mi = 8 >> t;
+            auto fk = std::make_tuple(K, mi);
+            if (!fwd_idx.count(fk)) {
+                fwd_idx[fk] = pl->fwd.size();
+                pl->fwd.push_back({K, mi, 0, {}, nullptr});
+            }
+            auto& fl = pl->fwd[fwd_idx[fk]];
+            fl.lds = std::max(fl.lds, fwd_lds_bytes(P, K));
+            for (int s0 = 0; s0 < S; s0 += K)
+                for (int c = g.tab_off[t]; c < g.tab_off[t + 1]; ++c) {
+                    const FwdChunk& ch = g.chunks_host[c];
+                    fl.items.push_back(FwdItem{i, ch.cls, ch.a0, ch.na, ch.b0, ch.nb, s0, 0});
+                }
+        }
         // backprojection + primal items: tiles x slice groups
         auto ak = std::make_tuple(K, P.dim, P.tgv, P.fuse_primal);
         if (!adj_idx.count(ak)) {
@@ -443,6 +536,7 @@ int plan_build(gr_plan* pl, const gr_geometry* const* geoms)
     }
     // largest chunks first, so the smallest fill the tail of the launch
     for (auto& l : pl->fwd) {
+        if (l.mi == 0) continue;  // of about one size, in the order of the images
         auto work = [&](const FwdItem& it) {
             const ProbDev& P = pl->probs[it.prob];
             return (double)it.na * it.nb * (it.cls == 0 ? P.nx : P.ny);
@@ -457,6 +551,7 @@ int plan_build(gr_plan* pl, const gr_geometry* const* geoms)
         }
     int rc = upload(pl->probs, &pl->probs_dev);
     for (auto& l : pl->fwd) if (!rc) rc = upload(l.items, &l.dev);
+    if (!rc) rc = upload(pl->tiles, &pl->tiles_dev);
     for (auto& l : pl->adj) if (!rc) rc = upload(l.items, &l.dev);
     for (auto& l : pl->dual) if (!rc) rc = upload(l.items, &l.dev);
     for (auto& l : pl->primal) if (!rc) rc = upload(l.items, &l.dev);
@@ -508,6 +603,10 @@ int plan_phase(gr_plan* pl, int phase, int fwd_mode, hipStream_t st)
                  : phase == 1 ? pl->fwd.size()
                  : phase == 2 ? pl->adj.size()
                               : pl->primal.size());
+    }
+    if (phase == PHASE_DUAL_FWD || phase == 1) {  // ahead of the fork
+        int rc = launch_transpose_batch(pl->probs_dev, pl->tiles_dev, (int)pl->tiles.size(), st);
+        if (rc) return rc;
     }
     const size_t nl = jobs.size();
     const int lanes = (int)std::min<size_t>(nl, gr_plan::PLAN_LANES);
@@ -563,8 +662,12 @@ int plan_phase(gr_plan* pl, int phase, int fwd_mode, hipStream_t st)
                                    l.tgv != 0, l.maxc, s);
         } else if (ph == 1) {
             const auto& l = pl->fwd[i];
-            rc = launch_fwd_batch(pl->probs_dev, l.dev, (int)l.items.size(), l.K, l.mi, l.lds,
-                                  fwd_mode, s);
+            if (l.mi == 0)
+                rc = launch_fwd_line_batch(pl->probs_dev, l.dev, (int)l.items.size(), l.K,
+                                           l.waves, fwd_mode, s);
+            else
+                rc = launch_fwd_batch(pl->probs_dev, l.dev, (int)l.items.size(), l.K, l.mi, l.lds,
+                                      fwd_mode, s);
         } else if (ph == 2) {
             const auto& l = pl->adj[i];
             rc = launch_adj_batch(pl->probs_dev, l.dev, (int)l.items.size(), l.K, l.dim,
@@ -678,6 +781,8 @@ int gr_geometry_create(const float* ofs, int na, int nx, int ny, int nd, gr_geom
     g.adj_tile_y = std::max(nx, ny) <= 256 ? 16 : 32;
     g.fuse_primal = 0;
     g.ofs_dev = nullptr; g.fwd_dev = nullptr; g.chunks_dev = nullptr;
+    g.shear_dev = nullptr; g.lines_dev = nullptr; g.line0_dev = nullptr; g.bins_dev = nullptr;
+    g.shear_stride = g.shear_waves = 0;
     std::vector<FwdAngle> fa(na);
     for (int j = 0; j < na; ++j) {
         const double c = ofs[4 * j], s = ofs[4 * j + 1], o = ofs[4 * j + 2];
@@ -706,6 +811,8 @@ int gr_geometry_create(const float* ofs, int na, int nx, int ny, int nd, gr_geom
         g.chunks_host.insert(g.chunks_host.end(), c.begin(), c.end());
     }
     g.tab_off[4] = (int)g.chunks_host.size();
+    ShearTables sh;
+    const bool sheared = make_shear(fa, nd, std::max(nx, ny) + SHEAR_BLOCK, sh);
     hipError_t e = hipMalloc(&g.ofs_dev, sizeof(float) * 4 * na);
     if (e == hipSuccess) e = hipMalloc(&g.fwd_dev, sizeof(FwdAngle) * na);
     if (e == hipSuccess) e = hipMalloc(&g.chunks_dev, sizeof(FwdChunk) * g.chunks_host.size());
@@ -721,6 +828,31 @@ int gr_geometry_create(const float* ofs, int na, int nx, int ny, int nd, gr_geom
         gr_geometry_destroy(gg);
         return rc;
     }
+    if (sheared) {
+        g.shear_stride = std::max(nx, ny) + SHEAR_BLOCK;
+        for (int a = 0; a < na; ++a)
+            g.shear_waves = std::max(g.shear_waves, (sh.line0[a + 1] - sh.line0[a] + 63) / 64);
+        // one allocation and one copy for the four tables
+        std::vector<char> all;
+        auto put = [&](const auto& v) {
+            const size_t at = all.size(), n = sizeof(v[0]) * v.size();
+            all.resize((at + n + 63) / 64 * 64);
+            std::memcpy(all.data() + at, v.data(), n);
+            return at;
+        };
+        put(sh.shear);
+        const size_t lines = put(sh.lines), line0 = put(sh.line0), bins = put(sh.bins);
+        char* dev = nullptr;
+        int rc = upload(all, &dev);
+        g.shear_dev = reinterpret_cast<Shear*>(dev);
+        if (rc) {
+            gr_geometry_destroy(gg);
+            return rc;
+        }
+        g.lines_dev = reinterpret_cast<FwdLine*>(dev + lines);
+        g.line0_dev = reinterpret_cast<int*>(dev + line0);
+        g.bins_dev = reinterpret_cast<FwdBin*>(dev + bins);
+    }
     *out = gg;
     return GR_OK;
 }
@@ -732,6 +864,7 @@ int gr_geometry_destroy(gr_geometry* gg)
     if (g.ofs_dev) (void)hipFree(g.ofs_dev);
     if (g.fwd_dev) (void)hipFree(g.fwd_dev);
     if (g.chunks_dev) (void)hipFree(g.chunks_dev);
+    if (g.shear_dev) (void)hipFree(g.shear_dev);
     delete gg;
     return GR_OK;
 }

@@ -48,6 +48,24 @@ struct FwdChunk {
     int cls, a0, na, b0, nb, pad0, pad1, pad2;
 };
 
+// Tables of the sheared forward projection.  An item follows the line
+// candidate = j + s(l) through the image, s(l) = rint(-l mstep / mcand), along
+// which the detector coordinate is j mcand + off + d(l), |d| <= |mcand| / 2.
+struct Shear {
+    float d;
+    int s;
+};
+struct FwdLine {
+    int j;
+    float rel;  // j mcand + off - m, m the nearest bin
+};
+// Items that reach a bin: `first`, relative to the angle's first item, and in
+// `code` three bits per item: 0 past the last, 1 / 2 / 3 for m = bin + 1 / bin
+// / bin - 1.
+constexpr int FWD_BIN_ITEMS = 6;
+struct FwdBin {
+    int first, code;
+};
 // Everything a kernel needs to know about one reconstruction problem (or one
 // standalone projector call): sizes, derived scalars, geometry tables and
 // device state.  Passed by value for single problems and through a device
@@ -59,6 +77,13 @@ struct ProbDev {
     int fwd_band, fwd_pitch, adj_tile_y, adj_segw, adj_achunk, fuse_primal;
     const float4* ofs;     // na x (cos, sin, off, 1/cos)
     const FwdAngle* fwd;   // na, sorted by class
+    // sheared projection: na x shear_stride (lines), items, per angle its
+    // first item, na x nd bins
+    const Shear* shear;
+    const FwdLine* lines;
+    const int* line0;
+    const FwdBin* bins;
+    int shear_stride;
     // state; for standalone projector calls: ubar = image in, ku = sinogram
     // out (forward), lam = sinogram in, ktl = image out (backprojection)
     float *u, *ubar, *p, *pbar, *v, *w, *lam, *ktl, *ku;
@@ -82,6 +107,9 @@ struct AdjItem { int prob, x0, y0, s0; };
 // z + nz * channel (primal step).
 struct DualItem { int prob, x0, y0, z; };
 
+constexpr int SHEAR_BLOCK = 8;       // lines per table read
+constexpr double FWD_SHEAR_MIN = 0.7;
+
 // Device-side geometry (owned by gr_geometry).
 struct Geometry {
     int nx, ny, nd, na;
@@ -91,6 +119,14 @@ struct Geometry {
     int tab_off[5];          // table t = chunks [tab_off[t], tab_off[t+1]),
                              // built for 8, 4, 2, 1 items per thread
     std::vector<FwdChunk> chunks_host;
+    // sheared projection (every |mcand| in [FWD_SHEAR_MIN, 1], i.e. unit
+    // detector bins); otherwise null.  One allocation, owned by shear_dev
+    Shear* shear_dev;        // na x shear_stride
+    FwdLine* lines_dev;
+    int* line0_dev;          // na + 1
+    FwdBin* bins_dev;        // na x nd
+    int shear_stride;
+    int shear_waves;         // waves of items of the angle with the most
     int fwd_band;            // lines per LDS band (0: automatic)
     int adj_tile_y;          // rows per backprojection tile
     int fuse_primal;         // 1: primal step in the backprojection epilogue
@@ -102,7 +138,37 @@ struct Geometry {
 // iteration (two-stream schedule): fewer, larger work-groups.
 // FWD_AUTOBAND: the geometry's band height is automatic, so a launch beside
 // the dual step may size it for its grid.
-enum { FWD_WRITE = 1, FWD_KL = 2, FWD_L2 = 4, FWD_PROX = 8, FWD_BESIDE = 16, FWD_AUTOBAND = 32 };
+// FWD_SCRATCH: P.ktl (as large as the image) may be overwritten: inside an
+// iteration, where the backprojection fills it afterwards.
+enum {
+    FWD_WRITE = 1, FWD_KL = 2, FWD_L2 = 4, FWD_PROX = 8, FWD_BESIDE = 16, FWD_AUTOBAND = 32,
+    FWD_SCRATCH = 64
+};
+
+// A batch problem's descriptor.  The pointers of a descriptor read from memory
+// are generic to the compiler, which would access them by flat instructions
+// (slower, and counted with LDS: a wait for one is a wait for all); they are
+// global.  The cast goes through an integer, or it is folded away.  10 batch
+// iterations of 64 mixed slices: 10.68 ms before, 10.49 ms with it.
+template <class T>
+__device__ __forceinline__ T* as_global(T* p)
+{
+    return (T*)(__attribute__((address_space(1))) T*)(uintptr_t)p;
+}
+__device__ __forceinline__ ProbDev load_prob(const ProbDev* __restrict__ probs, int i)
+{
+    ProbDev P = probs[i];
+    P.ofs = as_global(P.ofs); P.fwd = as_global(P.fwd);
+    P.shear = as_global(P.shear); P.lines = as_global(P.lines);
+    P.line0 = as_global(P.line0); P.bins = as_global(P.bins);
+    P.u = as_global(P.u); P.ubar = as_global(P.ubar); P.p = as_global(P.p);
+    P.pbar = as_global(P.pbar); P.v = as_global(P.v); P.w = as_global(P.w);
+    P.lam = as_global(P.lam); P.ktl = as_global(P.ktl); P.ku = as_global(P.ku);
+    P.f = as_global(P.f); P.mfac = as_global(P.mfac);
+    P.halo_ubar_hi = as_global(P.halo_ubar_hi); P.halo_pbar_lo = as_global(P.halo_pbar_lo);
+    P.halo_v_lo = as_global(P.halo_v_lo); P.halo_w_hi = as_global(P.halo_w_hi);
+    return P;
+}
 
 // Loads / stores of arrays a stencil kernel streams once, with the
 // non-temporal hint when NT: single problems whose state outgrows the
@@ -164,6 +230,12 @@ __device__ __forceinline__ int stencil_block()
     return ((local / G) * 8 + xcd) * G + local % G;
 }
 
+inline void set_shear(ProbDev& P, const Geometry& g)
+{
+    P.shear = g.shear_dev; P.lines = g.lines_dev; P.line0 = g.line0_dev; P.bins = g.bins_dev;
+    P.shear_stride = g.shear_stride;
+}
+
 // Kernel-side sizes derived from a problem and its tuning.
 int fwd_pitch_of(int nx, int ny);
 int fwd_table_choice(const Geometry& g, long long groups, double wg_per_cu = 3.0);
@@ -199,6 +271,20 @@ int launch_primal_part(const ProbDev& P, int part, hipStream_t st);
 // ---- launchers (batches: descriptor table + item table) -------------------
 int launch_fwd_batch(const ProbDev* probs_dev, const FwdItem* items, int nitems, int K,
                      int mi, size_t lds, int mode, hipStream_t st);
+// The sheared forward projection of batch problems: items {prob, J, first
+// angle, angles, 0, 0, s0} of K slices, J = waves of items of one angle and
+// angles * J <= waves; after launch_transpose_batch (items: 32 x 32 tiles x0,
+// y0 of slice z).  With FWD_LINE_WAVES waves the forward phase of 64 mixed
+// slices (96^2 to 384^2) takes 0.45 ms; with 9, 10 and 16: 0.58, 0.56, 0.54
+// (a multiple of 4 loads the SIMDs evenly, and 16 leave room for one
+// work-group less); one launch per J 0.48.
+constexpr int FWD_LINE_WAVES = 12;
+int launch_fwd_line_batch(const ProbDev* probs_dev, const FwdItem* items, int nitems, int K,
+                          int waves, int mode, hipStream_t st);
+int launch_transpose_batch(const ProbDev* probs_dev, const DualItem* items, int nitems,
+                           hipStream_t st);
+// Whether an iteration of this problem projects forward by lines.
+bool fwd_by_lines(const ProbDev& P, const Geometry& g);
 int launch_adj_batch(const ProbDev* probs_dev, const AdjItem* items, int nitems, int K,
                      int dim, bool tgv, bool primal, size_t lds, hipStream_t st);
 int launch_primal_batch(const ProbDev* probs_dev, const DualItem* items, int nitems, int dim,

@@ -76,6 +76,228 @@ __device__ __forceinline__ void lds_store(float* sh, int pos, const float (&v)[K
     }
 }
 
+// Sinogram epilogue of the projection by lines, K slices s0.. at (angle id,
+// bin i): store and/or apply the prox (2D:316-338).  The gather has its own
+// copy: called from there, this costs its schedule 3%.
+template <int K>
+__device__ __forceinline__ void fwd_epilogue(const ProbDev& P, int mode, int s0, int id, int i,
+                                             const float (&val)[K])
+{
+    const int nslices = P.nz * P.nch;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const int s = s0 + k;
+        if (s >= nslices) continue;
+        const size_t idx = ((size_t)s * P.na + id) * P.nd + i;
+        if (mode & FWD_WRITE) P.ku[idx] = val[k];
+        if (mode & FWD_KL) {
+            const float m = P.mfac[s / P.nz];
+            const float sv = P.lam[idx] + P.sigma_p * val[k];
+            const float z = sv - m;
+            const float d = z * z + 4.f * P.sigma_p * P.f[idx] * m;
+            P.lam[idx] = sv - 0.5f * (z + sqrtf(d));
+        } else if (mode & FWD_L2) {
+            const float m = P.mfac[s / P.nz];
+            P.lam[idx] = (P.lam[idx] + P.sigma_p * (val[k] - P.f[idx])) * m;
+        }
+    }
+}
+
+// --------------------------------------------------------------------------
+// Sheared forward projection (unit detector bins).  At line l of the stepping
+// axis, candidate c = j + s(l) has detector coordinate
+//   t = l mstep + c mcand + off = (j mcand + off) + d(l),  |d| <= |mcand| / 2,
+// so along a fixed j the coordinate stays within one bin of the integer m
+// nearest to j mcand + off.  An item (one lane) follows one j through the
+// lines and, with v = t - m in [-1, 1], sums its hat-weighted contributions
+// max(-v, 0) img to bin m - 1, (1 - |v|) img to m and max(v, 0) img to m + 1.
+// (Sums of img, v img and |v| img, combined at the end, save two operations
+// an item and line and no time, and cost a bit of precision.)  Neighbouring lanes read neighbouring
+// pixels of a line, and s(l), d(l) are scalars of the wave, so lines are read
+// from memory directly (no LDS, no barriers): rows of the image for class 1,
+// rows of its transpose (P.ktl) for class 0.
+//
+// A work-group holds angles [a0, a0 + count) of K slices: for each J waves of
+// items, times ns = 1 or 2: one wave for both halves of the lines, or one for
+// each.  At the end the items' sums go through LDS, the halves are added, and
+// every bin adds its items in the order of j; so neither K, ns nor a batch
+// changes a value.
+//
+// What it replaces for stacks of few slices (the gather below) stages bands
+// of lines in LDS behind barriers and finds each ray's candidates from the
+// ray, 5 operations and a read for each of 3 candidates; with a work-group or
+// less per CU its time is that chain's latency.  Here a line costs an item
+// one read and 3 operations, in flight 8 at a time.  Bound by the L1's rate
+// (about 8 cycles a wave's read) and, for single slices, by latency; two
+// halves give single slices twice the waves (317 x 317 x 3, 71 angles, 10
+// iterations: 1000 us with one wave, 898 with two; 183 x 183: 680, 630).
+// --------------------------------------------------------------------------
+typedef int ShearOct __attribute__((ext_vector_type(2 * SHEAR_BLOCK), aligned(4)));
+typedef const __attribute__((address_space(4))) ShearOct* ShearOctPtr;
+
+template <int K>
+__device__ __forceinline__ void fwd_line_body(const ProbDev& P, int a0, int count, int s0, int J,
+                                              int ns, int mode, float* sh)
+{
+    if (mode & FWD_PROX) mode |= P.disc == GR_DISC_KL ? FWD_KL : FWD_L2;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int job = wave % J, run = wave / J % ns, al = wave / (J * ns);
+    const int a = a0 + min(al, count - 1);
+    const FwdAngle A = P.fwd[a];
+    const int first = P.line0[a], n = P.line0[a + 1] - first;
+    const int nline = A.cls == 0 ? P.nx : P.ny, ncand = A.cls == 0 ? P.ny : P.nx;
+    const int last = P.nz * P.nch - 1;
+    const float* __restrict__ img[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+        img[k] = (A.cls == 0 ? P.ktl : P.ubar) + (size_t)min(s0 + k, last) * ((size_t)nline * ncand);
+
+    // sums of the first and the second half of the lines, in this order
+    // whichever waves take them; `part` is [angle][3][K][item]
+    const int items = J * 64, i = job * 64 + lane;
+    float* part = sh + (size_t)al * 3 * K * items;
+    float acc[3][K];
+    for (int half = run; half < 2; half += ns) {
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
+#pragma unroll
+            for (int k = 0; k < K; ++k) acc[m][k] = 0.f;
+        if (job * 64 < n && al < count) {
+            const FwdLine L = P.lines[first + min(job * 64 + lane, n - 1)];
+            const int jf = __builtin_amdgcn_readfirstlane(L.j), jl = __builtin_amdgcn_readlane(L.j, 63);
+            const int blocks = (nline + SHEAR_BLOCK - 1) / SHEAR_BLOCK;
+            const int b0 = blocks * half / 2, b1 = blocks * (half + 1) / 2;
+            const ShearOctPtr table = (ShearOctPtr)(P.shear + (size_t)a * P.shear_stride);
+            ShearOct next = table[b0];
+            for (int b = b0; b < b1; ++b) {
+                const ShearOct q = next;
+                if (b + 1 < b1) next = table[b + 1];
+                const int l0 = b * SHEAR_BLOCK;
+                // candidates of the block's lines (s is monotonic along them)
+                const int lo = jf + min(q[1], q[2 * SHEAR_BLOCK - 1]);
+                const int hi = jl + max(q[1], q[2 * SHEAR_BLOCK - 1]);
+                if (hi < 0 || lo >= ncand) continue;
+                float p[SHEAR_BLOCK][K];
+                if (lo >= 0 && hi < ncand && l0 + SHEAR_BLOCK <= nline) {
+#pragma unroll
+                    for (int l = 0; l < SHEAR_BLOCK; ++l) {
+                        const unsigned at = (unsigned)(L.j + ((l0 + l) * ncand + q[2 * l + 1]));
+#pragma unroll
+                        for (int k = 0; k < K; ++k) p[l][k] = img[k][at];
+                    }
+                } else {  // zero beyond the image
+#pragma unroll
+                    for (int l = 0; l < SHEAR_BLOCK; ++l) {
+                        const int c = L.j + q[2 * l + 1];
+                        const bool in = c >= 0 && c < ncand && l0 + l < nline;
+                        const unsigned at = in ? (unsigned)((l0 + l) * ncand + c) : 0u;
+#pragma unroll
+                        for (int k = 0; k < K; ++k) {
+                            const float v = img[k][at];
+                            p[l][k] = in ? v : 0.f;
+                        }
+                    }
+                }
+#pragma unroll
+                for (int l = 0; l < SHEAR_BLOCK; ++l) {
+                    const float v = L.rel + __int_as_float(q[2 * l]);
+                    const float hi1 = fmaxf(v, 0.f), lo1 = hi1 - v, mid = 1.f - fabsf(v);
+#pragma unroll
+                    for (int k = 0; k < K; ++k) {
+                        acc[0][k] = fmaf(lo1, p[l][k], acc[0][k]);
+                        acc[1][k] = fmaf(mid, p[l][k], acc[1][k]);
+                        acc[2][k] = fmaf(hi1, p[l][k], acc[2][k]);
+                    }
+                }
+            }
+        }
+        if (half == 0 && al < count) {
+#pragma unroll
+            for (int m = 0; m < 3; ++m)
+#pragma unroll
+                for (int k = 0; k < K; ++k) part[(m * K + k) * items + i] = acc[m][k];
+        }
+    }
+    if (ns > 1) __syncthreads();
+    if (run == ns - 1 && al < count) {
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
+#pragma unroll
+            for (int k = 0; k < K; ++k) part[(m * K + k) * items + i] += acc[m][k];
+    }
+    __syncthreads();
+    if (al >= count) return;
+    // the angle's bins, by its J ns waves
+    for (int b = (run * J + job) * 64 + lane; b < P.nd; b += J * ns * 64) {
+        const FwdBin B = P.bins[(size_t)a * P.nd + b];
+        float val[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) val[k] = 0.f;
+#pragma unroll
+        for (int r = 0; r < FWD_BIN_ITEMS; ++r) {
+            const int c = ((B.code >> (3 * r)) & 7) - 1;
+            if (c < 0) continue;
+#pragma unroll
+            for (int k = 0; k < K; ++k) val[k] += part[(c * K + k) * items + B.first + r];
+        }
+        fwd_epilogue<K>(P, mode, s0, A.id, b, val);
+    }
+}
+
+template <int K>
+__global__ __launch_bounds__(1024) void fwd_line_kernel(ProbDev P, int J, int ns, int mode)
+{
+    extern __shared__ float sh[];
+    const int work = xcd_work_id(blockIdx.x, gridDim.x);
+    fwd_line_body<K>(P, work % P.na, 1, (work / P.na) * K, J, ns, mode, sh);
+}
+
+template <int K>
+__global__ __launch_bounds__(1024) void fwd_line_batch_kernel(const ProbDev* __restrict__ probs,
+                                                              const FwdItem* __restrict__ items,
+                                                              int mode)
+{
+    extern __shared__ float sh[];
+    const FwdItem I = items[xcd_work_id(blockIdx.x, gridDim.x)];
+    const ProbDev P = load_prob(probs, I.prob);
+    fwd_line_body<K>(P, I.a0, I.na, I.s0, I.cls, 1, mode, sh);
+}
+
+// P.ktl = slice s of P.ubar transposed, one 32 x 32 tile through LDS.
+__device__ __forceinline__ void transpose_tile(const ProbDev& P, int s, int x0, int y0)
+{
+    __shared__ float tile[32][33];
+    const int nx = P.nx, ny = P.ny, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    const float* __restrict__ src = P.ubar + (size_t)s * nx * ny;
+    float* __restrict__ dst = P.ktl + (size_t)s * nx * ny;
+#pragma unroll
+    for (int r = 0; r < 32; r += 8) {
+        const int x = x0 + tx, y = y0 + ty + r;
+        if (x < nx && y < ny) tile[ty + r][tx] = src[(size_t)y * nx + x];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 32; r += 8) {
+        const int x = x0 + ty + r, y = y0 + tx;
+        if (x < nx && y < ny) dst[(size_t)x * ny + y] = tile[tx][ty + r];
+    }
+}
+
+__global__ __launch_bounds__(256) void transpose_kernel(ProbDev P, int tiles_x, int tiles_y)
+{
+    const int tiles = tiles_x * tiles_y, t = blockIdx.x % tiles;
+    transpose_tile(P, blockIdx.x / tiles, 32 * (t % tiles_x), 32 * (t / tiles_x));
+}
+
+__global__ __launch_bounds__(256) void transpose_batch_kernel(const ProbDev* __restrict__ probs,
+                                                              const DualItem* __restrict__ items)
+{
+    const DualItem I = items[blockIdx.x];
+    const ProbDev P = load_prob(probs, I.prob);
+    transpose_tile(P, I.z, I.x0, I.y0);
+}
+
 // --------------------------------------------------------------------------
 // Forward projection of one work item: K slices s0.. (sharing all geometry)
 // times a chunk of (angle, bin) items whose angles step along the same axis.
@@ -258,7 +480,7 @@ __global__ __launch_bounds__(FWD_THREADS) void fwd_batch_kernel(const ProbDev* _
     // items are sorted largest first; plain block order deals them
     // round-robin over the XCDs, which balances the load
     const FwdItem I = items[blockIdx.x];
-    const ProbDev P = probs[I.prob];
+    const ProbDev P = load_prob(probs, I.prob);
     fwd_body<K, MI>(P, I, mode, sh);
 }
 
@@ -357,7 +579,7 @@ __global__ __launch_bounds__(DUAL_BX* DUAL_BY) void primal_batch_kernel(
     const ProbDev* __restrict__ probs, const DualItem* __restrict__ items)
 {
     const DualItem I = items[blockIdx.x];
-    const ProbDev P = probs[I.prob];
+    const ProbDev P = load_prob(probs, I.prob);
     primal_body<DIM, TGV, PART>(P, I);
 }
 
@@ -491,7 +713,7 @@ __global__ __launch_bounds__(ADJ_THREADS) void adj_batch_kernel(const ProbDev* _
 {
     extern __shared__ float sh[];
     const AdjItem I = items[xcd_work_id(blockIdx.x, gridDim.x)];
-    const ProbDev P = probs[I.prob];
+    const ProbDev P = load_prob(probs, I.prob);
     adj_body<K, PRIMAL, DIM, TGV>(P, I, sh);
 }
 
@@ -635,9 +857,63 @@ static int fwd_single_k(const ProbDev& Pin, const Geometry& g, int nslices, int 
     return GR_OK;
 }
 
+// Where an iteration projects by lines: it needs the shear tables, angles of
+// at most 16 waves, and P.ktl to hold the transposed slices (with the
+// primal step fused into the backprojection it stays as it is).  Iteration time by lines
+// relative to the gather (TGV, 4 channels, 60 angles), for N x N x S slices:
+//   N = 96: S 4 1 / 1.2, 64 1.10; 128: 32 1 / 1.26, 128 1 / 1.02, 256 1.10;
+//   200: 32 1 / 1.42, 80 1 / 1.04; 256: 8 1 / 2.2, 32 1 / 1.55, 64 1.00,
+//   128 1.18; 384: 32 1 / 1.35; 512: 16 1 / 1.9, 64 1 / 1.05;
+//   one channel, one slice: N = 48 1.06, 96 1 / 1.05, 183 1 / 1.6, 512 1 / 4.
+// With many slices the gather's work-groups leave registers and LDS for the
+// dual step beside them, and these leave it waiting.
+bool fwd_by_lines(const ProbDev& P, const Geometry& g)
+{
+    const long long S = (long long)P.nz * P.nch, px = (long long)P.nx * P.ny;
+    return g.shear_dev && g.shear_waves <= 16 && !P.fuse_primal && px >= 6400 && S <= 64 &&
+           256 * S <= px;
+}
+
+// LDS bytes of a work-group of that many waves (one or two runs of lines)
+static size_t fwd_line_lds(int K, int waves)
+{
+    return (size_t)3 * K * waves * 64 * sizeof(float);
+}
+
+template <int K>
+static int fwd_line_k(const ProbDev& P, const Geometry& g, int nslices, int mode, hipStream_t st)
+{
+    const int groups = (nslices + K - 1) / K, J = g.shear_waves;
+    const int ns = J <= 8 ? 2 : 1;
+    const int tx = (P.nx + 31) / 32, ty = (P.ny + 31) / 32;
+    const long long tiles = (long long)tx * ty * nslices, blocks = (long long)groups * P.na;
+    if (tiles > 0x7fffffff || blocks > 0x7fffffff) {
+        set_error("radon: invalid grid (%lld blocks)", std::max(tiles, blocks));
+        return GR_ERR_INVALID;
+    }
+    hipLaunchKernelGGL(transpose_kernel, dim3((unsigned)tiles), dim3(256), 0, st, P, tx, ty);
+    hipLaunchKernelGGL((fwd_line_kernel<K>), dim3((unsigned)blocks), dim3(64 * J * ns),
+                       fwd_line_lds(K, J), st, P, J, ns, mode);
+    GR_LAUNCH_CHECK("fwd_line_kernel");
+    return GR_OK;
+}
+
 int launch_fwd(const ProbDev& P, const Geometry& g, int nslices, int mode, hipStream_t st)
 {
     if (nslices <= 0) return GR_OK;
+    if ((mode & FWD_SCRATCH) && fwd_by_lines(P, g)) {
+        // fewer slices per work-group where angles x groups would not give
+        // every CU one: 317 x 317 x 3, 71 angles, 10 iterations 1000 / 932 /
+        // 898 us with 4 / 2 / 1 (71, 142 and 213 work-groups); 199 x 199 x 42,
+        // 45 angles, 5 iterations 483 / 521 / 605 us (495 work-groups and up)
+        int K = slice_group(nslices);
+        while (K > 1 && (long long)((nslices + K - 1) / K) * P.na < 256) K /= 2;
+        switch (K) {
+        case 4: return fwd_line_k<4>(P, g, nslices, mode, st);
+        case 2: return fwd_line_k<2>(P, g, nslices, mode, st);
+        default: return fwd_line_k<1>(P, g, nslices, mode, st);
+        }
+    }
     switch (slice_group(nslices)) {
     case 4: return fwd_single_k<4>(P, g, nslices, mode, st);
     case 2: return fwd_single_k<2>(P, g, nslices, mode, st);
@@ -866,6 +1142,32 @@ int launch_fwd_batch(const ProbDev* probs, const FwdItem* items, int nitems, int
 #undef GR_FB_K
 #undef GR_FB
     GR_LAUNCH_CHECK("fwd_batch_kernel");
+    return GR_OK;
+}
+
+int launch_transpose_batch(const ProbDev* probs, const DualItem* items, int nitems,
+                           hipStream_t st)
+{
+    if (nitems <= 0) return GR_OK;
+    hipLaunchKernelGGL(transpose_batch_kernel, dim3((unsigned)nitems), dim3(256), 0, st, probs,
+                       items);
+    GR_LAUNCH_CHECK("transpose_batch_kernel");
+    return GR_OK;
+}
+
+int launch_fwd_line_batch(const ProbDev* probs, const FwdItem* items, int nitems, int K,
+                          int waves, int mode, hipStream_t st)
+{
+    if (nitems <= 0) return GR_OK;
+    const dim3 grd((unsigned)nitems), blk(64 * waves);
+    const size_t lds = fwd_line_lds(K, waves);
+    if (K == 4)
+        hipLaunchKernelGGL((fwd_line_batch_kernel<4>), grd, blk, lds, st, probs, items, mode);
+    else if (K == 2)
+        hipLaunchKernelGGL((fwd_line_batch_kernel<2>), grd, blk, lds, st, probs, items, mode);
+    else
+        hipLaunchKernelGGL((fwd_line_batch_kernel<1>), grd, blk, lds, st, probs, items, mode);
+    GR_LAUNCH_CHECK("fwd_line_batch_kernel");
     return GR_OK;
 }
 

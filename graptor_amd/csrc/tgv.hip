@@ -503,7 +503,7 @@ __global__ __launch_bounds__(DUAL_BX* DUAL_BY) void dual_batch_kernel(
     const ProbDev* __restrict__ probs, const DualItem* __restrict__ items)
 {
     const DualItem I = items[blockIdx.x];
-    const ProbDev P = probs[I.prob];
+    const ProbDev P = load_prob(probs, I.prob);
     dual_body<DIM, CPL, TGV, MAXC>(P, I);
 }
 
@@ -523,7 +523,7 @@ __global__ __launch_bounds__(DUAL_BX* DUAL_BY) void dual_wide_batch_kernel(
     const ProbDev* __restrict__ probs, const DualItem* __restrict__ items)
 {
     const DualItem I = items[blockIdx.x];
-    const ProbDev P = probs[I.prob];
+    const ProbDev P = load_prob(probs, I.prob);
     dual_body_wide<DIM, CPL, TGV>(P, I);
 }
 
