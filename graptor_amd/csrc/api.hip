@@ -202,6 +202,7 @@ ProbDev make_prob(const gr_geometry* gg, const gr_tgv_params* p, const gr_tgv_st
     P.fwd_pitch = fwd_pitch_of(g.nx, g.ny);
     P.fwd_band = g.fwd_band > 0 ? g.fwd_band : fwd_band_auto(P.fwd_pitch, K);
     P.adj_tile_y = g.adj_tile_y;
+    P.narrow_bins = g.narrow_bins;
     P.adj_segw = adj_segw_of(P.adj_tile_y);
     P.adj_achunk = adj_achunk_of(g.na, P.adj_segw, K);
     P.fuse_primal = g.fuse_primal;
@@ -723,6 +724,7 @@ ProbDev standalone(const gr_geometry* gg, int nslices)
     P.fwd = g.fwd_dev;
     P.fwd_band = g.fwd_band;
     P.adj_tile_y = g.adj_tile_y;
+    P.narrow_bins = g.narrow_bins;
     return P;
 }
 
@@ -783,9 +785,11 @@ int gr_geometry_create(const float* ofs, int na, int nx, int ny, int nd, gr_geom
     g.ofs_dev = nullptr; g.fwd_dev = nullptr; g.chunks_dev = nullptr;
     g.shear_dev = nullptr; g.lines_dev = nullptr; g.line0_dev = nullptr; g.bins_dev = nullptr;
     g.shear_stride = g.shear_waves = 0;
+    g.narrow_bins = 0;
     std::vector<FwdAngle> fa(na);
     for (int j = 0; j < na; ++j) {
         const double c = ofs[4 * j], s = ofs[4 * j + 1], o = ofs[4 * j + 2];
+        if (std::hypot(c, s) > 1.0 + 1e-5) g.narrow_bins = 1;
         FwdAngle a{};
         a.cls = std::fabs(s) >= std::fabs(c) ? 0 : 1;
         const double mc = a.cls == 0 ? s : c;

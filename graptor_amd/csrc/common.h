@@ -84,6 +84,7 @@ struct ProbDev {
     const int* line0;
     const FwdBin* bins;
     int shear_stride;
+    int narrow_bins;       // a step of one pixel may cross more than one bin
     // state; for standalone projector calls: ubar = image in, ku = sinogram
     // out (forward), lam = sinogram in, ktl = image out (backprojection)
     float *u, *ubar, *p, *pbar, *v, *w, *lam, *ktl, *ku;
@@ -129,6 +130,7 @@ struct Geometry {
     int shear_waves;         // waves of items of the angle with the most
     int fwd_band;            // lines per LDS band (0: automatic)
     int adj_tile_y;          // rows per backprojection tile
+    int narrow_bins;         // detector width below one pixel
     int fuse_primal;         // 1: primal step in the backprojection epilogue
 };
 

@@ -695,6 +695,73 @@ __device__ __forceinline__ void adj_body(const ProbDev& P, const AdjItem& I, flo
     }
 }
 
+// Backprojection of 64 x 4 pixels of K slices, bins read from memory: the
+// positions, weights and order of the tile the pixels belong to (y0 a multiple
+// of 4, tile_y as well), so the same bits.  For stacks that leave most CUs
+// without a tile: four to eight times the waves, no staging between barriers,
+// and 8 angles' reads in flight.  Bound by the latency of these reads; 183 x
+// 183, 90 angles 32 us by tiles, 9.8 so; 317 x 317 x 3, 71 angles 43 and 16.
+template <int K>
+__device__ __forceinline__ void adj_direct_body(const ProbDev& P, const AdjItem& I)
+{
+    __shared__ float4 par[ADJ_THREADS];
+    const int nx = P.nx, ny = P.ny, nd = P.nd, na = P.na;
+    const int last = P.nz * P.nch - 1, tile_y = P.adj_tile_y;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int x = I.x0 + lane, y = I.y0 + wv, ty0 = I.y0 / tile_y * tile_y;
+    const float xf = (float)x, yf = (float)y;
+    const size_t slice = (size_t)na * nd;
+    const float* __restrict__ sino[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) sino[k] = P.lam + (size_t)min(I.s0 + k, last) * slice;
+    float acc[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) acc[k] = 0.f;
+    for (int a0 = 0; a0 < na; a0 += ADJ_THREADS) {
+        const int A = min(ADJ_THREADS, na - a0);
+        __syncthreads();
+        if (tid < A) {
+            const float4 o = P.ofs[a0 + tid];
+            const float tmin = o.z + (float)I.x0 * o.x + (float)ty0 * o.y +
+                               fminf(0.f, (float)(ADJ_TX - 1) * o.x) +
+                               fminf(0.f, (float)(tile_y - 1) * o.y);
+            const int lo = (int)floorf(tmin) - 1;
+            par[tid] = make_float4(o.x, o.y, o.z - (float)lo, __int_as_float(lo));
+        }
+        __syncthreads();
+#pragma unroll 8
+        for (int al = 0; al < A; ++al) {
+            const float4 pa = par[al];
+            const float t = fmaf(yf, pa.y, fmaf(xf, pa.x, pa.z));
+            const float p = __builtin_amdgcn_fractf(t);
+            const float q = 1.f - p;
+            const int i = __float_as_int(pa.w) + (int)t;
+            const bool in0 = (unsigned)i < (unsigned)nd, in1 = (unsigned)(i + 1) < (unsigned)nd;
+            const unsigned row = (unsigned)((a0 + al) * nd);
+            const unsigned e0 = row + (in0 ? i : 0), e1 = row + (in1 ? i + 1 : 0);
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                const float g0 = sino[k][e0], g1 = sino[k][e1];
+                acc[k] = fmaf(p, in1 ? g1 : 0.f, fmaf(q, in0 ? g0 : 0.f, acc[k]));
+            }
+        }
+    }
+    if (x >= nx || y >= ny) return;
+    const size_t plane = (size_t)nx * ny;
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+        if (I.s0 + k <= last) P.ktl[(size_t)(I.s0 + k) * plane + (size_t)y * nx + x] = acc[k];
+}
+
+template <int K>
+__global__ __launch_bounds__(ADJ_THREADS) void adj_direct_kernel(ProbDev P, int tiles_x,
+                                                                 int ntiles)
+{
+    const int work = xcd_work_id(blockIdx.x, gridDim.x), tile = work % ntiles;
+    adj_direct_body<K>(P, AdjItem{0, tile % tiles_x * ADJ_TX, tile / tiles_x * 4,
+                                  (work / ntiles) * K});
+}
+
 template <int K, bool PRIMAL, int DIM, bool TGV, int MAXR>
 __global__ __launch_bounds__(ADJ_THREADS) void adj_single_kernel(ProbDev P, int tiles_x,
                                                                  int ntiles)
@@ -977,6 +1044,17 @@ static int adj_single_k(const ProbDev& Pin, int nslices, bool primal, hipStream_
     return GR_OK;
 }
 
+template <int K>
+static int adj_direct_k(const ProbDev& P, int nslices, hipStream_t st)
+{
+    const int tiles_x = (P.nx + ADJ_TX - 1) / ADJ_TX, ntiles = tiles_x * ((P.ny + 3) / 4);
+    const int groups = (nslices + K - 1) / K;
+    hipLaunchKernelGGL((adj_direct_kernel<K>), dim3((unsigned)(groups * ntiles)),
+                       dim3(ADJ_THREADS), 0, st, P, tiles_x, ntiles);
+    GR_LAUNCH_CHECK("adj_direct_kernel");
+    return GR_OK;
+}
+
 int launch_adj(const ProbDev& P, int nslices, bool primal, hipStream_t st, bool beside)
 {
     if (nslices <= 0) return GR_OK;
@@ -986,8 +1064,28 @@ int launch_adj(const ProbDev& P, int nslices, bool primal, hipStream_t st, bool 
     // slices of accumulators per lane: 2.92 against 2.47 ms on 512^2 x 1024
     // slices, 90 angles), nor beside the dual step (0.7874 against 0.7860 ms
     // per two-stream iteration).
-    if (nslices >= 8 && !primal && !beside && P.adj_tile_y <= 16)
-        return adj_single_k<8>(P, nslices, primal, st);
+    const bool wide = nslices >= 8 && !primal && !beside && P.adj_tile_y <= 16;
+    // Where the tiles would not give every CU a work-group, a small stack is
+    // read directly, in at most 6144 waves and with as few slices per wave as
+    // that allows.  One call, 60 angles, us with 1 / 2 / 4 slices a wave
+    // against tiles: 64 x 64 x 1 12.5 to 20, x 64 12.6 / 12.2 / 12.4 to 32;
+    // 183 x 183 x 3 12 to 22, x 16 21 / 19 / 19 to 32, x 64 (288 work-groups)
+    // 64 / 49 / 43 to 37; 256 x 256 x 24 (192) 46 / 36 / 32 to 33, x 32 (256)
+    // 58 / 45 / 39 to 33; 512 x 512 x 1 12 to 33, x 4 31 / 25 / 24 to 35.
+    // Whole iterations: 183 x 183 x 16 71 to 78, 512 x 512 x 4 94 to 109, but
+    // 64 x 64 x 256 (256 work-groups) 89 to 86, 256 x 256 x 24 (384) 116 to 108.
+    // Bins narrower than a pixel stay with the tiles at every size.
+    if (!primal && !P.narrow_bins && P.adj_tile_y >= 4 && P.adj_tile_y % 4 == 0) {
+        const long long cols = (P.nx + ADJ_TX - 1) / ADJ_TX, rows = cols * P.ny;
+        const long long tiles = cols * ((P.ny + P.adj_tile_y - 1) / P.adj_tile_y);
+        const int K = wide ? 8 : slice_group(nslices);
+        if (tiles * ((nslices + K - 1) / K) < 256) {
+            if (rows * nslices <= 6144) return adj_direct_k<1>(P, nslices, st);
+            if (rows * ((nslices + 1) / 2) <= 6144) return adj_direct_k<2>(P, nslices, st);
+            if (rows * ((nslices + 3) / 4) <= 6144) return adj_direct_k<4>(P, nslices, st);
+        }
+    }
+    if (wide) return adj_single_k<8>(P, nslices, primal, st);
     switch (slice_group(nslices)) {
     case 4: return adj_single_k<4>(P, nslices, primal, st);
     case 2: return adj_single_k<2>(P, nslices, primal, st);
