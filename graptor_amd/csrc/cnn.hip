@@ -228,6 +228,208 @@ __global__ __launch_bounds__(256) void conv_tile_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// 3x3 convolution of TM output rows at once.  The tile above reads one or two
+// LDS fragments per MFMA and is bound by them (one row, 32 output channels: 64
+// LDS cycles a CU for 32 MFMA cycles) and by staging three rows and the
+// weights for one row of outputs.  Here a wave keeps the weight fragments of
+// a channel chunk in registers, reads each fragment of a staged row once for
+// the up to three output rows it serves, and stages TM + 2 rows for TM.  Per
+// output the order is that of the tile (chunk, vertical, horizontal tap, k
+// step), so are the bits.  Weights are the A operand: a lane then holds
+// consecutive channels of a pixel and stores 16 bytes at a time.
+//
+// U-Net of 32 images of 256 x 256, all 3x3 layers: 2366 us by tiles, 1440 so
+// (32 output channels at 256 x 256: 212 to 139 us a layer; 64 at 128 x 128:
+// 142 to 104; 128 at 64 x 64 and 256 at 32 x 32: 161 to 78); 700 GFLOP, 580 us
+// at the rate of a large product.  Two output tiles per wave (TN = 2) need
+// spills at 4 rows: 64 x 64 85 instead of 78 us.  What bounds it now: one or
+// two work-groups per CU, whose staging is not all hidden, and at 256 x 256 memory
+// (1.3 GB, 277 us at 4.6 TB/s, of 556).
+// ---------------------------------------------------------------------------
+template <int WAVES_M_, int TM_, int TN_, int KC_>
+struct ConvRows {
+    static constexpr int WAVES_M = WAVES_M_, TM = TM_, TN = TN_, KC = KC_;
+    static constexpr int WAVES_N = 4 / WAVES_M;
+    static constexpr int MP = WAVES_M * 32;       // pixels of a row per work-group
+    static constexpr int NC = WAVES_N * TN * 32;  // output channels per work-group
+    static constexpr int AS = KC + 8;             // LDS halves per staged pixel
+    static constexpr int R = TM + 2, P = MP + 2;  // staged rows and pixels of a row
+    static constexpr int G = KC / 8, KS = KC / 16;
+    static constexpr int NA = (R * P * G + 255) / 256;
+    static constexpr size_t lds_bytes = 2 * (size_t)R * P * AS;
+};
+
+template <class T>
+__device__ __forceinline__ void conv_rows_load(u32x4 (&ra)[T::NA], const uint16_t* __restrict__ x,
+                                               int ldx, int cx0, int c0, int tid, int row, int img,
+                                               int x0, int H, int W, int cin)
+{
+#pragma unroll
+    for (int k = 0; k < T::NA; ++k) {
+        const int e = tid + 256 * k, g = e % T::G, q = e / T::G, pp = q % T::P, r = q / T::P;
+        const int yy = row + r - 1, xx = x0 + pp - 1, c = c0 + 8 * g;
+        const bool ok = r < T::R && yy >= 0 && yy < H && xx >= 0 && xx < W && c < cin;
+        ra[k] = ok ? *reinterpret_cast<const u32x4*>(x + ((size_t)(img * H + yy) * W + xx) * ldx +
+                                                      cx0 + c)
+                   : u32x4{0u, 0u, 0u, 0u};
+    }
+}
+
+// Weight fragments of one vertical offset and one chunk, read where they lie
+// (zero beyond cin and cout, both multiples of the fragment).
+template <class T>
+__device__ __forceinline__ void conv_rows_weights(bf16x8 (&wf)[3][T::KS][T::TN],
+                                                  const uint16_t* __restrict__ w, int dy, int c0,
+                                                  int co0, int lane, int cin, int cout)
+{
+#pragma unroll
+    for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+        for (int k = 0; k < T::KS; ++k)
+#pragma unroll
+            for (int j = 0; j < T::TN; ++j) {
+                const int co = co0 + 32 * j, c = c0 + 16 * k;
+                U16x8 v = {{0, 0, 0, 0, 0, 0, 0, 0}};
+                if (co < cout && c < cin)
+                    v = *reinterpret_cast<const U16x8*>(
+                        w + ((size_t)(co + (lane & 31)) * 9 + 3 * dy + dx) * cin + c +
+                        8 * (lane >> 5));
+                wf[dx][k][j] = as_bf16x8(v);
+            }
+}
+
+template <int WAVES_M, int TM, int TN, int KC>
+__global__ __launch_bounds__(256, 2) void conv_rows_kernel(
+    const uint16_t* __restrict__ x, int ldx, int cx0, const uint16_t* __restrict__ w,
+    const float* __restrict__ bias, void* __restrict__ y, int ldy, int cy0, int H, int W,
+    int cin, int cout, int relu, int out_f32, int vec)
+{
+    using T = ConvRows<WAVES_M, TM, TN, KC>;
+    constexpr int AS = T::AS, P = T::P, R = T::R, G = T::G, KS = T::KS;
+    extern __shared__ __attribute__((aligned(16))) uint16_t lds[];  // [R][P][AS]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = lane >> 5, l32 = lane & 31;
+    const int segs = (W + T::MP - 1) / T::MP, co_blocks = (cout + T::NC - 1) / T::NC;
+    const int row_tiles = (H + TM - 1) / TM;
+    int b = xcd_work_id(blockIdx.x, gridDim.x);
+    const int cob = b % co_blocks;
+    b /= co_blocks;
+    const int seg = b % segs;
+    b /= segs;
+    const int row = b % row_tiles * TM, img = b / row_tiles;
+    const int x0 = seg * T::MP;
+    const int wm = wave % WAVES_M, wn = wave / WAVES_M;
+    const int co0 = cob * T::NC + wn * TN * 32;
+
+    floatx16 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+    u32x4 ra[T::NA];
+    bf16x8 wf[3][3][KS][TN];
+    conv_rows_load<T>(ra, x, ldx, cx0, 0, tid, row, img, x0, H, W, cin);
+#pragma unroll
+    for (int dy = 0; dy < 3; ++dy) conv_rows_weights<T>(wf[dy], w, dy, 0, co0, lane, cin, cout);
+    for (int c0 = 0; c0 < cin; c0 += KC) {
+        const bool more = c0 + KC < cin;
+        __syncthreads();  // the previous chunk is no longer read
+#pragma unroll
+        for (int k = 0; k < T::NA; ++k) {
+            const int e = tid + 256 * k;
+            if (e < R * P * G)
+                *reinterpret_cast<u32x4*>(lds + (size_t)(e / G) * AS + 8 * (e % G)) = ra[k];
+        }
+        __syncthreads();
+        if (more)  // in flight during this chunk's MFMAs
+            conv_rows_load<T>(ra, x, ldx, cx0, c0 + KC, tid, row, img, x0, H, W, cin);
+        const uint16_t* px = lds + (size_t)(wm * 32 + l32) * AS + 8 * h;
+#pragma unroll
+        for (int s = 0; s < R; ++s) {
+            U16x8 a[3][KS];
+#pragma unroll
+            for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+                for (int k = 0; k < KS; ++k)
+                    a[dx][k] = *reinterpret_cast<const U16x8*>(px + (size_t)(s * P + dx) * AS +
+                                                               16 * k);
+#pragma unroll
+            for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+                for (int k = 0; k < KS; ++k)
+#pragma unroll
+                    for (int dy = 0; dy < 3; ++dy) {
+                        const int i = s - dy;
+                        if (i < 0 || i >= TM) continue;
+#pragma unroll
+                        for (int j = 0; j < TN; ++j)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                                wf[dy][dx][k][j], as_bf16x8(a[dx][k]), acc[i][j], 0, 0, 0);
+                    }
+            // this vertical offset is done with the chunk
+            if (s >= TM - 1 && more)
+                conv_rows_weights<T>(wf[s - (TM - 1)], w, s - (TM - 1), c0 + KC, co0, lane, cin,
+                                     cout);
+        }
+    }
+    // epilogue: lane holds pixel l32, channels 8(r/4) + 4h + r%4 of each tile
+    const int xo = x0 + wm * 32 + l32;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        const int cb = co0 + 32 * j;
+        if (cb >= cout) continue;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            if (row + i >= H) continue;
+            const size_t pix = (size_t)(img * H + row + i) * W + xo;
+            float v[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                v[r] = acc[i][j][r] + (bias ? bias[cb + 8 * (r >> 2) + 4 * h + (r & 3)] : 0.f);
+                if (relu) v[r] = v[r] > 0.f ? v[r] : 0.f;
+            }
+            if (vec) {
+                // pairs of groups of 4 channels: exchanged between the halves
+                // of the wave, h = 0 holds channels 16 q .. + 7, h = 1 the next 8
+                uint16_t* o = reinterpret_cast<uint16_t*>(y) + pix * ldy + cy0 + cb;
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    uint32_t lo[2], hi[2];
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        lo[e] = f2bf(v[8 * q + 2 * e]) |
+                                (uint32_t)f2bf(v[8 * q + 2 * e + 1]) << 16;
+                        hi[e] = f2bf(v[8 * q + 4 + 2 * e]) |
+                                (uint32_t)f2bf(v[8 * q + 4 + 2 * e + 1]) << 16;
+                    }
+                    u32x4 out;
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        const auto p = __builtin_amdgcn_permlane32_swap(lo[e], hi[e], false, false);
+                        out[e] = p[0];
+                        out[2 + e] = p[1];
+                    }
+                    if (xo < W) *reinterpret_cast<u32x4*>(o + 16 * q + 8 * h) = out;
+                }
+            } else if (xo < W) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const size_t at = pix * ldy + cy0 + cb + 8 * (r >> 2) + 4 * h + (r & 3);
+                    if (out_f32)
+                        reinterpret_cast<float*>(y)[at] = v[r];
+                    else
+                        reinterpret_cast<uint16_t*>(y)[at] = f2bf(v[r]);
+                }
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Weight gradient: dW[co][tap][ci] += sum over pixels of
 // dy[p][co] * x[p shifted by tap][ci].  M = co (32 per wave), N = ci (32 per
 // wave), K = pixels.  A work-group covers 64 co x 64 ci and one row of taps
@@ -698,6 +900,32 @@ static void conv_tile_launch(const uint16_t* x, int ldx, int cx0, const uint16_t
                            cin, cout, relu, out_f32);
 }
 
+// Launches the row kernel with 4 or 2 rows a work-group, the most that give
+// every CU a work-group and waste few rows; false if neither does.  With 256,
+// inference of n images of 256 x 256: n = 2 333 us (347 by tiles alone, 333 at
+// 128, 356 at 64), n = 4 398 (453, 395, 379), n = 8 535 with two rows where
+// four are too many (576 without, 740 by tiles), n = 1 299 (298, 312, 323).
+template <int WAVES_M, int TM, int KC>
+static bool conv_rows_launch(const uint16_t* x, int ldx, int cx0, const uint16_t* w,
+                             const float* bias, void* y, int ldy, int cy0, int n, int H, int W,
+                             int cin, int cout, int relu, int out_f32, hipStream_t st)
+{
+    using T = ConvRows<WAVES_M, TM, 1, KC>;
+    const long long blocks = (long long)n * ((H + TM - 1) / TM) * ((W + T::MP - 1) / T::MP) *
+                             ((cout + T::NC - 1) / T::NC);
+    if (blocks < 256 || blocks > 0x7fffffff || (H % TM != 0 && H < 2 * TM)) {
+        if constexpr (TM > 2)
+            return conv_rows_launch<WAVES_M, TM / 2, KC>(x, ldx, cx0, w, bias, y, ldy, cy0, n, H,
+                                                         W, cin, cout, relu, out_f32, st);
+        return false;
+    }
+    const int vec = !out_f32 && vec8(cout, ldy, cy0, y);
+    hipLaunchKernelGGL((conv_rows_kernel<WAVES_M, TM, 1, KC>), dim3((unsigned)blocks), dim3(256),
+                       T::lds_bytes, st, x, ldx, cx0, w, bias, y, ldy, cy0, H, W, cin, cout, relu,
+                       out_f32, vec);
+    return true;
+}
+
 extern "C" {
 
 int gr_cnn_conv_fwd(const void* x, int ldx, int cx0, const void* w, const float* bias, void* y,
@@ -714,6 +942,24 @@ int gr_cnn_conv_fwd(const void* x, int ldx, int cx0, const void* w, const float*
     const hipStream_t st = cnn_stream(stream);
     const uint16_t* xp = (const uint16_t*)x;
     const uint16_t* wp = (const uint16_t*)w;
+    // 3x3: rows of 32, 64 or 128 pixels with 128, 64 or 32 output channels; the
+    // channels of a chunk are those of the tile below, in the same order (16
+    // instead of 32 where there are no more)
+    bool rows = false;
+#define GR_ROWS(...)                                                                          \
+    rows = conv_rows_launch<__VA_ARGS__>(xp, ldx, cx0, wp, bias, y, ldy, cy0, n, H, W, cin,   \
+                                         cout, relu, out_f32, st)
+    if (taps == 9) {
+        if (W <= 64 && cout % 128 == 0) GR_ROWS(1, 4, 16);
+        else if (cout % 64 == 0) GR_ROWS(2, 4, 32);
+        else if (cin <= 16) GR_ROWS(4, 4, 16);
+        else GR_ROWS(4, 4, 32);
+    }
+#undef GR_ROWS
+    if (rows) {
+        GR_LAUNCH_CHECK("conv_rows_kernel");
+        return GR_OK;
+    }
     if (W <= 32 && cout % 256 == 0)
         conv_tile_launch<1, 1, 2, 16>(xp, ldx, cx0, wp, bias, y, ldy, cy0, n, H, W, cin, cout,
                                       taps, relu, out_f32, st);

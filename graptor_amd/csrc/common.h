@@ -147,6 +147,16 @@ enum {
     FWD_SCRATCH = 64
 };
 
+// Map hardware block order (dealt round-robin over the 8 XCDs) to a work
+// order in which consecutive work ids run on the same XCD and share its L2.
+__device__ __forceinline__ int xcd_work_id(int bid, int nb)
+{
+    const int xcd = bid & 7, local = bid >> 3;
+    const int per = nb >> 3, rem = nb & 7;
+    return (xcd < rem) ? xcd * (per + 1) + local
+                       : rem * (per + 1) + (xcd - rem) * per + local;
+}
+
 // A batch problem's descriptor.  The pointers of a descriptor read from memory
 // are generic to the compiler, which would access them by flat instructions
 // (slower, and counted with LDS: a wait for one is a wait for all); they are
