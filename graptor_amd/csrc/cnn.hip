@@ -431,105 +431,168 @@ __global__ __launch_bounds__(256, 2) void conv_rows_kernel(
 
 // ---------------------------------------------------------------------------
 // Weight gradient: dW[co][tap][ci] += sum over pixels of
-// dy[p][co] * x[p shifted by tap][ci].  M = co (32 per wave), N = ci (32 per
-// wave), K = pixels.  A work-group covers 64 co x 64 ci and one row of taps
-// (the three taps of one vertical offset, or the single 1x1 tap) over a chunk
-// of rows; per 64-pixel step it stages dy as [co][px] and the input row as
-// [shift][ci][px] (one copy per horizontal shift, so every MFMA operand is
-// an aligned 16-byte LDS read), then runs 4 k steps x the row's taps.
-// Partial sums go to the FP32 accumulator with atomics (split-K over the
-// chunks).
+// dy[p][co] * x[p shifted by tap][ci].  M = 32 co, N = 32 ci, K = pixels, all
+// taps in one wave (9 x 16 accumulators).  A wave walks down the rows of a
+// segment of SEG pixels with the last three rows of x in LDS, so a step stages
+// one row of dy and one of x.  MFMA fragments run along pixels, memory along
+// channels: a lane loads 8 pixels x 8 channels, transposes them in registers
+// (one byte permute per pair of pixels) and writes 16 bytes of pixels a
+// channel.  x starts one pixel early, so the fragments of the three
+// horizontal taps come out of 10 consecutive pixels: as read, shifted by a
+// half, shifted by a dword.  Waves share nothing until the end, when the
+// work-group's four are summed and added to the FP32 result by atomics.
+//
+// A training step on 16 images of 256 x 256, all 14 3x3 layers: 1860 us with
+// scalar transposing LDS writes, one copy per horizontal tap, and one vertical
+// tap a work-group; 850 so (350 GFLOP: 290 at the rate of a large product).
+// Bound by staging (a wave hides the next row's loads behind one row's 36
+// MFMAs, two waves a SIMD) and, for few images, by the sums at the end.
 // ---------------------------------------------------------------------------
-constexpr int WG_PX = 64;            // pixels per staged step (4 MFMA k steps)
-constexpr int WG_LD = WG_PX + 8;     // LDS row stride (halves): conflict-free fragment reads
-
-template <int TAPS>
-__global__ __launch_bounds__(256) void conv_wgrad_kernel(
+template <int TAPS, int SEG>
+__global__ __launch_bounds__(256, 2) void conv_wgrad_kernel(
     const uint16_t* __restrict__ x, int ldx, int cx0, const uint16_t* __restrict__ dy, int ldd,
-    int cd0, float* __restrict__ dw, int n, int H, int W, int cin, int cout, int rows_per_chunk)
+    int cd0, float* __restrict__ dw, int n, int H, int W, int cin, int cout, int rows)
 {
-    constexpr int NS = TAPS == 9 ? 3 : 1;  // horizontal shifts = taps per work-group
-    __shared__ __attribute__((aligned(16))) uint16_t sdy[64][WG_LD];      // [co][px]
-    __shared__ __attribute__((aligned(16))) uint16_t sx[NS][64][WG_LD];   // [shift][ci][px]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    constexpr int NR = TAPS == 9 ? 3 : 1, HALO = NR / 2;
+    constexpr int PITCH = SEG + 8;              // halves of a channel: conflict-free fragments
+    constexpr int ROW = 32 * PITCH;             // one staged row of 32 channels
+    constexpr int WAVE = (1 + NR) * ROW;        // dy, ring of x
+    constexpr int LDS = 4 * WAVE > 4 * NR * 2048 ? 4 * WAVE : 4 * NR * 2048;
+    __shared__ __attribute__((aligned(16))) uint16_t lds[LDS];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = lane >> 5, l32 = lane & 31;
-    const int co_blocks = (cout + 63) / 64, ci_blocks = (cin + 63) / 64;
-    int b = blockIdx.x;
-    const int cob = b % co_blocks; b /= co_blocks;
-    const int cib = b % ci_blocks; b /= ci_blocks;
-    const int trow = b % NS; b /= NS;  // vertical offset index (3x3) or 0 (1x1)
-    const int chunk = b;               // chunk of rows over all images
-    const int total_rows = n * H;
-    const int r0 = chunk * rows_per_chunk;
-    const int r1 = min(total_rows, r0 + rows_per_chunk);
-    const int dyo = TAPS == 9 ? trow - 1 : 0;
-    const int wm = wave & 1, wn = wave >> 1;
+    const int co_blocks = (cout + 31) / 32, ci_blocks = (cin + 31) / 32;
+    const int segs = (W + SEG - 1) / SEG, row_chunks = (H + rows - 1) / rows;
+    int b = xcd_work_id(blockIdx.x, gridDim.x);
+    const int cob = b % co_blocks * 32;
+    b /= co_blocks;
+    const int cib = b % ci_blocks * 32;
+    b /= ci_blocks;
+    const int unit = 4 * b + wave;  // (image, segment, chunk of rows)
+    const int img = unit / (segs * row_chunks), us = unit - img * segs * row_chunks;
+    const int x0 = us / row_chunks * SEG, r0 = us % row_chunks * rows;
+    const int nrows = img < n ? min(rows, H - r0) : 0;
 
-    floatx16 acc[NS];
+    // staging role: 8 pixels (block j) x 8 channels (group g) of dy or of x
+    const int kind = lane / (SEG / 2), sub = lane % (SEG / 2), g = sub & 3, j = sub >> 2;
+    const bool is_x = kind == 1;
+    const int ch = (is_x ? cib : cob) + 8 * g;
+    const int px0 = x0 + 8 * j - (is_x ? HALO : 0);
+    const int ld = is_x ? ldx : ldd;
+    const uint16_t* __restrict__ src = (is_x ? x + cx0 : dy + cd0) + ch;
+    const bool ch_ok = kind < 2 && ch < (is_x ? cin : cout);
+    uint16_t* my = lds + wave * WAVE;
+    u32x4 v[8], ve[2];  // ve: the two pixels of x after the last block
+    auto load = [&](int t) {
+        const int row = r0 + t + (is_x ? HALO : 0);
+        const bool ok = ch_ok && row >= 0 && row < H && t < nrows && (is_x || t >= 0);
+        const uint16_t* at = src + (size_t)(img * H + row) * W * ld;
 #pragma unroll
-    for (int d = 0; d < NS; ++d)
+        for (int i = 0; i < 8; ++i) {
+            const int px = px0 + i;
+            v[i] = ok && px >= 0 && px < W ? *reinterpret_cast<const u32x4*>(at + (size_t)px * ld)
+                                           : u32x4{0u, 0u, 0u, 0u};
+        }
+        if (HALO) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int px = px0 + 8 + i;
+                ve[i] = ok && is_x && j == SEG / 8 - 1 && px < W
+                            ? *reinterpret_cast<const u32x4*>(at + (size_t)px * ld)
+                            : u32x4{0u, 0u, 0u, 0u};
+            }
+        }
+    };
+    auto store = [&](int slot) {
+        uint16_t* to = my + (is_x ? (1 + slot) * ROW : 0) + 8 * g * PITCH + 8 * j;
+        if (kind < 2) {
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const uint32_t sel = c & 1 ? 0x07060302u : 0x05040100u;
+                u32x4 o;
+#pragma unroll
+                for (int p = 0; p < 4; ++p)
+                    o[p] = __builtin_amdgcn_perm(v[2 * p + 1][c / 2], v[2 * p][c / 2], sel);
+                *reinterpret_cast<u32x4*>(to + c * PITCH) = o;
+            }
+            if (HALO && is_x && j == SEG / 8 - 1) {
+#pragma unroll
+                for (int c = 0; c < 8; ++c)
+                    *reinterpret_cast<uint32_t*>(to + c * PITCH + 8) = __builtin_amdgcn_perm(
+                        ve[1][c / 2], ve[0][c / 2], c & 1 ? 0x07060302u : 0x05040100u);
+            }
+        }
+    };
+
+    floatx16 acc[TAPS];
+#pragma unroll
+    for (int d = 0; d < TAPS; ++d)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[d][r] = 0.f;
 
-    for (int gr_ = r0; gr_ < r1; ++gr_) {
-        const int img = gr_ / H, row = gr_ - img * H;
-        const int yy = row + dyo;
-        for (int x0 = 0; x0 < W; x0 += WG_PX) {
-            __syncthreads();
-            // dy: 64 px x 8 channel groups (two per thread)
+    // row t of dy meets rows t - 1, t, t + 1 of x, stored by steps t - 2, t - 1, t
+    int slot = 0;
+    if (nrows > 0) load(-2 * HALO);
+    for (int t = -2 * HALO; t < nrows; ++t) {
+        // the wave's own LDS operations complete in order; the compiler must
+        // keep them in order too
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        store(slot);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        load(t + 1);
+        if (t >= 0) {
 #pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                const int e = tid + 256 * k, p = e & 63, g = e >> 6;
-                const int xo = x0 + p, co = cob * 64 + 8 * g;
-                U16x8 v = {{0, 0, 0, 0, 0, 0, 0, 0}};
-                if (co < cout && xo < W)
-                    v = *reinterpret_cast<const U16x8*>(
-                        dy + ((size_t)(img * H + row) * W + xo) * ldd + cd0 + co);
+            for (int ks = 0; ks < SEG / 16; ++ks) {
+                const int at = l32 * PITCH + 16 * ks + 8 * h;
+                const bf16x8 a = as_bf16x8(*reinterpret_cast<const U16x8*>(my + at));
 #pragma unroll
-                for (int j = 0; j < 8; ++j) sdy[8 * g + j][p] = v.v[j];
-            }
-            // x: pixels x0 - 1 .. x0 + 64 of row yy (3x3) or x0 .. x0 + 63 (1x1),
-            // written once per horizontal shift they serve
-            constexpr int QP = TAPS == 9 ? WG_PX + 2 : WG_PX;
-            for (int e = tid; e < QP * 8; e += 256) {
-                const int q = e % QP, g = e / QP;
-                const int xs = x0 + q - (TAPS == 9 ? 1 : 0), ci = cib * 64 + 8 * g;
-                U16x8 v = {{0, 0, 0, 0, 0, 0, 0, 0}};
-                if (ci < cin && yy >= 0 && yy < H && xs >= 0 && xs < W)
-                    v = *reinterpret_cast<const U16x8*>(
-                        x + ((size_t)(img * H + yy) * W + xs) * ldx + cx0 + ci);
+                for (int ry = 0; ry < NR; ++ry) {
+                    const int sl = NR == 1 ? 0 : (slot + 1 + ry) % 3;
+                    const uint16_t* from = my + (1 + sl) * ROW + at;
+                    const u32x4 q = *reinterpret_cast<const u32x4*>(from);
+                    bf16x8 f;
+                    __builtin_memcpy(&f, &q, 16);
+                    acc[NR * ry] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, f, acc[NR * ry], 0, 0, 0);
+                    if constexpr (NR == 3) {
+                        const uint32_t q4 = *reinterpret_cast<const uint32_t*>(from + 8);
+                        const u32x4 two{q[1], q[2], q[3], q4};
+                        u32x4 one;
 #pragma unroll
-                for (int d = 0; d < NS; ++d) {
-                    const int p = q - d;  // shift d reads pixel x0 + p + d - 1
-                    if (p >= 0 && p < WG_PX) {
-#pragma unroll
-                        for (int j = 0; j < 8; ++j) sx[d][8 * g + j][p] = v.v[j];
+                        for (int i = 0; i < 4; ++i)
+                            one[i] = __builtin_amdgcn_alignbit(two[i], q[i], 16);
+                        __builtin_memcpy(&f, &one, 16);
+                        acc[3 * ry + 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            a, f, acc[3 * ry + 1], 0, 0, 0);
+                        __builtin_memcpy(&f, &two, 16);
+                        acc[3 * ry + 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            a, f, acc[3 * ry + 2], 0, 0, 0);
                     }
                 }
             }
-            __syncthreads();
-#pragma unroll
-            for (int ks = 0; ks < WG_PX / 16; ++ks) {
-                const U16x8 a =
-                    *reinterpret_cast<const U16x8*>(&sdy[wm * 32 + l32][ks * 16 + 8 * h]);
-#pragma unroll
-                for (int d = 0; d < NS; ++d) {
-                    const U16x8 bb =
-                        *reinterpret_cast<const U16x8*>(&sx[d][wn * 32 + l32][ks * 16 + 8 * h]);
-                    acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(a), as_bf16x8(bb),
-                                                                     acc[d], 0, 0, 0);
-                }
-            }
         }
+        slot = NR == 1 ? 0 : (slot == 2 ? 0 : slot + 1);
     }
-    const int ci = cib * 64 + wn * 32 + l32;
+
+    // sum of the four waves, NR taps at a time: [wave][tap][r][lane]
+    float* sums = reinterpret_cast<float*>(lds);
 #pragma unroll
-    for (int d = 0; d < NS; ++d) {
-        const int t = TAPS == 9 ? 3 * trow + d : 0;
+    for (int d0 = 0; d0 < TAPS; d0 += NR) {
+        __syncthreads();
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int co = cob * 64 + wm * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-            if (co < cout && ci < cin) atomicAdd(&dw[((size_t)co * TAPS + t) * cin + ci], acc[d][r]);
+        for (int d = 0; d < NR; ++d)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                sums[((wave * NR + d) * 16 + r) * 64 + lane] = acc[d0 + d][r];
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 4 * NR; ++k) {
+            const int e = 4 * k + wave, d = e / 16, r = e % 16;  // of this wave's lanes
+            float s = 0.f;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) s += sums[((u * NR + d) * 16 + r) * 64 + lane];
+            const int co = cob + 8 * (r >> 2) + 4 * h + (r & 3), ci = cib + l32;
+            if (co < cout && ci < cin) atomicAdd(&dw[((size_t)co * TAPS + d0 + d) * cin + ci], s);
         }
     }
 }
@@ -926,6 +989,27 @@ static bool conv_rows_launch(const uint16_t* x, int ldx, int cx0, const uint16_t
     return true;
 }
 
+template <int TAPS, int SEG>
+static void conv_wgrad_launch(const uint16_t* x, int ldx, int cx0, const uint16_t* dy, int ldd,
+                              int cd0, float* dw, int n, int H, int W, int cin, int cout,
+                              hipStream_t st)
+{
+    const long long tiles = (long long)((cout + 31) / 32) * ((cin + 31) / 32);
+    const long long columns = (long long)n * ((W + SEG - 1) / SEG);
+    // Rows per wave: long walks read x once and add fewer partial sums, but
+    // every CU should have work.  One work-group per CU, one and a half where
+    // that leaves long walks.  Training steps of n images of 256 x 256 with 256
+    // / 384 / 512 work-groups: n = 2 1162 / 1255 / 1292 us, n = 8 2003 / 1983 /
+    // 2095, n = 16 3215 / 3141 / 3215; with 128, n = 16 3451.
+    long long rows = columns * H * tiles / (4 * 256);
+    if (rows >= 12) rows = rows * 2 / 3;
+    rows = std::max<long long>(1, std::min<long long>(H, rows));
+    const long long units = columns * ((H + rows - 1) / rows);
+    hipLaunchKernelGGL((conv_wgrad_kernel<TAPS, SEG>), dim3((unsigned)(tiles * ((units + 3) / 4))),
+                       dim3(256), 0, st, x, ldx, cx0, dy, ldd, cd0, dw, n, H, W, cin, cout,
+                       (int)rows);
+}
+
 extern "C" {
 
 int gr_cnn_conv_fwd(const void* x, int ldx, int cx0, const void* w, const float* bias, void* y,
@@ -992,17 +1076,15 @@ int gr_cnn_conv_wgrad(const void* x, int ldx, int cx0, const void* dy, int ldd, 
         set_error("cnn_conv_wgrad: invalid arguments");
         return GR_ERR_INVALID;
     }
-    const int chunks = (n * H + rows_per_chunk - 1) / rows_per_chunk;
-    const long long blocks = (long long)((cout + 63) / 64) * ((cin + 63) / 64) *
-                             (taps == 9 ? 3 : 1) * chunks;
-    if (taps == 9)
-        hipLaunchKernelGGL(conv_wgrad_kernel<9>, dim3((unsigned)blocks), dim3(256), 0,
-                           cnn_stream(stream), (const uint16_t*)x, ldx, cx0, (const uint16_t*)dy,
-                           ldd, cd0, dw, n, H, W, cin, cout, rows_per_chunk);
+    const hipStream_t st = cnn_stream(stream);
+    const uint16_t* xp = (const uint16_t*)x;
+    const uint16_t* dp = (const uint16_t*)dy;
+    if (taps == 9 && W <= 32)
+        conv_wgrad_launch<9, 32>(xp, ldx, cx0, dp, ldd, cd0, dw, n, H, W, cin, cout, st);
+    else if (taps == 9)
+        conv_wgrad_launch<9, 64>(xp, ldx, cx0, dp, ldd, cd0, dw, n, H, W, cin, cout, st);
     else
-        hipLaunchKernelGGL(conv_wgrad_kernel<1>, dim3((unsigned)blocks), dim3(256), 0,
-                           cnn_stream(stream), (const uint16_t*)x, ldx, cx0, (const uint16_t*)dy,
-                           ldd, cd0, dw, n, H, W, cin, cout, rows_per_chunk);
+        conv_wgrad_launch<1, 64>(xp, ldx, cx0, dp, ldd, cd0, dw, n, H, W, cin, cout, st);
     GR_LAUNCH_CHECK("conv_wgrad_kernel");
     return GR_OK;
 }

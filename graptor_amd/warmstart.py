@@ -270,14 +270,9 @@ class UNet:
             if l.relu:
                 _lib.check(lib.gr_cnn_relu_bwd(dy.ptr, dy.ld, dy.c0, yout.ptr, yout.ld, yout.c0,
                                                dy.npix(), l.cout, st), "relu_bwd")
-            rows = n * xin.h
-            # work-groups per chunk: 64 x 64 channel tiles x rows of taps
-            blocks = ((l.cout + 63) // 64) * ((l.cin + 63) // 64) * (3 if l.taps == 9 else 1)
-            chunks = max(1, min(rows, 1024 // max(blocks, 1)))
-            rpc = max(1, (rows + chunks - 1) // chunks)
             _lib.check(lib.gr_cnn_conv_wgrad(xin.ptr, xin.ld, xin.c0, dy.ptr, dy.ld, dy.c0,
                                              self.g.data_ptr() + 4 * l.w_off, n, xin.h, xin.w,
-                                             l.cin, l.cout, l.taps, rpc, st), "wgrad")
+                                             l.cin, l.cout, l.taps, xin.h, st), "wgrad")
             _lib.check(lib.gr_cnn_bias_grad(dy.ptr, dy.ld, dy.c0, dy.npix(), l.cout,
                                             self.g.data_ptr() + 4 * l.b_off, st), "bias_grad")
             if dx is not None:

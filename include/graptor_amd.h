@@ -274,7 +274,8 @@ int gr_cnn_conv_fwd(const void *x, int ldx, int cx0, const void *w, const float 
                     int ldy, int cy0, int n, int H, int W, int cin, int cout, int taps, int relu,
                     int out_f32, void *stream);
 /* dw[co][tap][ci] += sum_pixels dy[p][co] x[p shifted by tap][ci] (FP32, atomic
- * split-K over chunks of rows_per_chunk image rows). */
+ * partial sums over chunks of image rows, whose number is chosen by the call;
+ * rows_per_chunk must be positive and is not used otherwise). */
 int gr_cnn_conv_wgrad(const void *x, int ldx, int cx0, const void *dy, int ldd, int cd0,
                       float *dw, int n, int H, int W, int cin, int cout, int taps,
                       int rows_per_chunk, void *stream);
