@@ -922,6 +922,28 @@ int gr_radon(const gr_geometry* gg, float* sino, const float* img, int nslices, 
     return launch_fwd(P, gg->g, nslices, FWD_WRITE, stream_of(stream));
 }
 
+size_t gr_radon_scratch_floats(const gr_geometry* gg, int nslices)
+{
+    if (!gg || nslices <= 0) return 0;
+    const ProbDev P = standalone(gg, nslices);
+    return fwd_by_lines(P, gg->g, true) ? (size_t)P.nx * P.ny * nslices : 0;
+}
+
+int gr_radon_scratch(const gr_geometry* gg, float* sino, const float* img, int nslices,
+                     float* scratch, void* stream)
+{
+    if (!gg || !sino || !img || nslices < 0 || !scratch || scratch == img) {
+        set_error("radon_scratch: invalid arguments");
+        return GR_ERR_INVALID;
+    }
+    ProbDev P = standalone(gg, nslices);
+    set_shear(P, gg->g);
+    P.ubar = const_cast<float*>(img);
+    P.ku = sino;
+    P.ktl = scratch;
+    return launch_fwd(P, gg->g, nslices, FWD_WRITE | FWD_SCRATCH | FWD_ALONE, stream_of(stream));
+}
+
 int gr_radon_ad(const gr_geometry* gg, float* img, const float* sino, int nslices, void* stream)
 {
     if (!gg || !sino || !img || nslices < 0) {

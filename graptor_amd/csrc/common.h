@@ -141,10 +141,11 @@ struct Geometry {
 // FWD_AUTOBAND: the geometry's band height is automatic, so a launch beside
 // the dual step may size it for its grid.
 // FWD_SCRATCH: P.ktl (as large as the image) may be overwritten: inside an
-// iteration, where the backprojection fills it afterwards.
+// iteration, where the backprojection fills it afterwards, or because the
+// caller says so.  FWD_ALONE: no dual step beside the launch.
 enum {
     FWD_WRITE = 1, FWD_KL = 2, FWD_L2 = 4, FWD_PROX = 8, FWD_BESIDE = 16, FWD_AUTOBAND = 32,
-    FWD_SCRATCH = 64
+    FWD_SCRATCH = 64, FWD_ALONE = 128
 };
 
 // Map hardware block order (dealt round-robin over the 8 XCDs) to a work
@@ -295,8 +296,9 @@ int launch_fwd_line_batch(const ProbDev* probs_dev, const FwdItem* items, int ni
                           int waves, int mode, hipStream_t st);
 int launch_transpose_batch(const ProbDev* probs_dev, const DualItem* items, int nitems,
                            hipStream_t st);
-// Whether an iteration of this problem projects forward by lines.
-bool fwd_by_lines(const ProbDev& P, const Geometry& g);
+// Whether an iteration of this problem (alone: a projection outside one)
+// projects forward by lines.
+bool fwd_by_lines(const ProbDev& P, const Geometry& g, bool alone = false);
 int launch_adj_batch(const ProbDev* probs_dev, const AdjItem* items, int nitems, int K,
                      int dim, bool tgv, bool primal, size_t lds, hipStream_t st);
 int launch_primal_batch(const ProbDev* probs_dev, const DualItem* items, int nitems, int dim,

@@ -914,21 +914,30 @@ static int fwd_single_k(const ProbDev& Pin, const Geometry& g, int nslices, int 
     return GR_OK;
 }
 
-// Where an iteration projects by lines: it needs the shear tables, angles of
-// at most 16 waves, and P.ktl to hold the transposed slices (with the
-// primal step fused into the backprojection it stays as it is).  Iteration time by lines
-// relative to the gather (TGV, 4 channels, 60 angles), for N x N x S slices:
-//   N = 96: S 4 1 / 1.2, 64 1.10; 128: 32 1 / 1.26, 128 1 / 1.02, 256 1.10;
-//   200: 32 1 / 1.42, 80 1 / 1.04; 256: 8 1 / 2.2, 32 1 / 1.55, 64 1.00,
-//   128 1.18; 384: 32 1 / 1.35; 512: 16 1 / 1.9, 64 1 / 1.05;
-//   one channel, one slice: N = 48 1.06, 96 1 / 1.05, 183 1 / 1.6, 512 1 / 4.
-// With many slices the gather's work-groups leave registers and LDS for the
-// dual step beside them, and these leave it waiting.
-bool fwd_by_lines(const ProbDev& P, const Geometry& g)
+// Where a call projects by lines: it needs the shear tables, angles of at most
+// 16 waves, and P.ktl to hold the transposed slices (with the primal step
+// fused into the backprojection it stays as it is).
+//
+// Alone, gather / by lines in us for N x N x S, 60 angles: N = 64: S 4 15 / 9,
+// 64 16 / 15, 128 17 / 23; 128: 1 20 / 11, 32 30 / 21, 64 33 / 32, 128 42 / 57;
+// 200: 4 63 / 16, 64 79 / 65, 128 101 / 107; 256: 4 90 / 19, 128 154 / 128,
+// 512 471 / 465; 512: 4 341 / 48, 64 683 / 245, 256 1069 / 1028; 180 angles:
+// N = 96: 4 21 / 14, 32 25 / 33; 200: 32 94 / 82, 64 148 / 146; 512: 128 1609 /
+// 1207: angles x groups of slices against pixels.
+//
+// In an iteration the gather shares the GPU with the dual step, for whose
+// work-groups it leaves room.  Time of an iteration by gather over that by
+// lines (TGV, 4 channels, 60 angles): N = 96: S 4 1.2, 64 0.91; 128: 32 1.26,
+// 128 1.02, 256 0.91; 200: 32 1.42, 80 1.04; 256: 8 2.2, 32 1.55, 64 1.00, 128
+// 0.85; 384: 32 1.35; 512: 16 1.9, 64 1.05; one slice: N = 48 0.94, 96 1.05,
+// 183 1.6, 512 4.
+bool fwd_by_lines(const ProbDev& P, const Geometry& g, bool alone)
 {
     const long long S = (long long)P.nz * P.nch, px = (long long)P.nx * P.ny;
-    return g.shear_dev && g.shear_waves <= 16 && !P.fuse_primal && px >= 6400 && S <= 64 &&
-           256 * S <= px;
+    const long long groups = (long long)P.na * ((S + 3) / 4);
+    if (!g.shear_dev || g.shear_waves > 16 || px < 6400) return false;
+    if (alone) return 24 * groups <= px && S * px <= (1ll << 25);
+    return !P.fuse_primal && S <= 64 && groups <= 960 && 17 * groups <= px;
 }
 
 // LDS bytes of a work-group of that many waves (one or two runs of lines)
@@ -958,7 +967,7 @@ static int fwd_line_k(const ProbDev& P, const Geometry& g, int nslices, int mode
 int launch_fwd(const ProbDev& P, const Geometry& g, int nslices, int mode, hipStream_t st)
 {
     if (nslices <= 0) return GR_OK;
-    if ((mode & FWD_SCRATCH) && fwd_by_lines(P, g)) {
+    if ((mode & FWD_SCRATCH) && fwd_by_lines(P, g, mode & FWD_ALONE)) {
         // fewer slices per work-group where angles x groups would not give
         // every CU one: 317 x 317 x 3, 71 angles, 10 iterations 1000 / 932 /
         // 898 us with 4 / 2 / 1 (71, 142 and 213 work-groups); 199 x 199 x 42,

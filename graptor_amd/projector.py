@@ -139,8 +139,25 @@ def radon(sino, img, r_struct, wait_for=None):
     ns_s, sv = _as_stack(sino, (g.na, g.nd), "radon sino")
     if ns_i != ns_s:
         raise ValueError(f"radon: {ns_i} image slices vs {ns_s} sinogram slices")
-    _lib.check(_lib.load().gr_radon(g.handle, sv.data_ptr(), imv.data_ptr(), ns_i,
-                                    _stream_ptr(img)), "radon")
+    lib = _lib.load()
+    tmp = _radon_scratch(lib.gr_radon_scratch_floats(g.handle, ns_i), img.device)
+    if tmp is not None:
+        _lib.check(lib.gr_radon_scratch(g.handle, sv.data_ptr(), imv.data_ptr(), ns_i,
+                                        tmp.data_ptr(), _stream_ptr(img)), "radon")
+        return
+    _lib.check(lib.gr_radon(g.handle, sv.data_ptr(), imv.data_ptr(), ns_i,
+                            _stream_ptr(img)), "radon")
+
+
+def _radon_scratch(n, device):
+    """``n`` floats of the current stream's memory (at most 128 MiB) for a small
+    stack; none while a graph is captured or where there is no memory left."""
+    if n == 0 or torch.cuda.is_current_stream_capturing():
+        return None
+    try:
+        return torch.empty(n, dtype=torch.float32, device=device)
+    except torch.cuda.OutOfMemoryError:
+        return None
 
 
 def radon_ad(img, sino, r_struct, wait_for=None):

@@ -24,7 +24,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .projector import RadonGeometry, make_function_feasible, radon, radon_ad
+from .projector import RadonGeometry, make_function_feasible, radon_ad
 from .solver import progress_line, resolve_device
 
 LSQR = 36.0
@@ -142,7 +142,9 @@ class SubsampledProblem:
             # fine pixel projects are zeroed in every slice
             ones = torch.ones((1, nd, nd), device=dev)
             r1 = torch.zeros((1, na1, nd), device=dev)
-            radon(r1, ones, self.g1)
+            # by the gather, like make_function_feasible: compared with zero
+            _lib.check(_lib.load().gr_radon(self.g1.handle, r1.data_ptr(), ones.data_ptr(), 1,
+                                            self._stream()), "radon")
             dead = (r1[0, :, :min(nd, nd1)] <= 0)
             if bool(dead.any()):
                 f1[:, :, :, :min(nd, nd1)].masked_fill_(dead.view(1, 1, na1, -1), 0.0)
@@ -191,10 +193,15 @@ class SubsampledProblem:
         return ctypes.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)
 
     # K = (R0 u0, S R1 u1) and its adjoint, on device tensors
-    def _forward(self, img, k0, k1_fine, k1):
-        C0, C1, nz, nd = self.C0, self.C1, self.nz, self.nd
-        radon(k0.view(C0 * nz, self.na0, nd), img[:C0].reshape(C0 * nz, nd, nd), self.g0)
-        radon(k1_fine.view(C1 * nz, self.na1, nd), img[C0:].reshape(C1 * nz, nd, nd), self.g1)
+    def _forward(self, img, k0, k1_fine, k1, scratch):
+        """``scratch``: as large as img, overwritten."""
+        C0, C1, nz = self.C0, self.C1, self.nz
+        lib, st = _lib.load(), self._stream()
+        for g, k, part, tmp in ((self.g0, k0, img[:C0], scratch[:C0]),
+                                (self.g1, k1_fine, img[C0:], scratch[C0:])):
+            if part.shape[0]:
+                _lib.check(lib.gr_radon_scratch(g.handle, k.data_ptr(), part.data_ptr(),
+                                                part.shape[0] * nz, tmp.data_ptr(), st), "radon")
         self.S.apply(k1_fine, k1, self.na1, C1, self._stream())
 
     def _adjoint(self, l0, l1, l1_fine, out):
@@ -224,7 +231,7 @@ class SubsampledProblem:
         for _ in range(rounds):
             nrm = self._norm(x)
             x.mul_(1.0 / nrm)
-            self._forward(x, k0, k1f, k1)
+            self._forward(x, k0, k1f, k1, y)  # K^T K x lands in y afterwards
             self._adjoint(k0, k1, l1f, y)
             x, y = y, x
         return math.sqrt(nrm)
@@ -242,7 +249,7 @@ class SubsampledProblem:
         with torch.cuda.device(self.device):
             for _ in range(int(n)):
                 _lib.check(lib.gr_tgv_dual_step(self.g0.handle, prm, state, st), "dual_step")
-                self._forward(self.ubar, self.ku0, self.ku1_fine, self.ku1)
+                self._forward(self.ubar, self.ku0, self.ku1_fine, self.ku1, self.ktl)
                 _lib.check(lib.gr_prox(disc, sp, mf0.data_ptr(), self.C0, per0,
                                        self.ku0.data_ptr(), self.f0.data_ptr(),
                                        self.lam0.data_ptr(), st), "prox")

@@ -63,3 +63,22 @@ def test_batch_gives_the_bits_of_each_problem():
     for c, (a, b) in enumerate(zip(alone, mixed)):
         assert torch.equal(a.ku, b.ku), CASES[c][:3]
         assert torch.equal(a.u, b.u), CASES[c][:3]
+
+
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_projection_with_scratch(case):
+    """The same cases outside an iteration; the image is left alone."""
+    from graptor_amd import _lib, radon
+    prob, u0 = _problem(case)
+    g, nx, ny, nd = prob.geometry, *CASES[case][:3]
+    S = u0.shape[0] * u0.shape[1]
+    img = torch.as_tensor(u0, device="cuda").reshape(S, ny, nx)
+    sino = torch.empty((S, g.na, nd), device="cuda")
+    radon(sino, img, (g, (nx, ny), (nd, g.na)))
+    want = O.radon_fwd(u0.astype(np.float64), g.ofs.T, nd).reshape(S, g.na, nd)
+    assert rel(sino.cpu().numpy(), want) <= BAR
+    assert np.array_equal(img.cpu().numpy().reshape(u0.shape), u0)
+    n = _lib.load().gr_radon_scratch_floats(g.handle, S)
+    assert n in (0, S * nx * ny)
+    assert _lib.load().gr_radon_scratch(g.handle, sino.data_ptr(), img.data_ptr(), S,
+                                        img.data_ptr(), None) == _lib.GR_ERR_INVALID
