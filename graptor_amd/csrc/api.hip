@@ -332,6 +332,13 @@ int iterate_single(const gr_geometry* gg, const ProbDev& P, int n_iter, int ku_o
             rc = launch_fwd(P, gg->g, nsl,
                             fwd_mode(it) | FWD_BESIDE | (gg->g.fwd_band > 0 ? 0 : FWD_AUTOBAND),
                             st);
+        // few slices: one launch for both (the dual step is over before the
+        // forward projection is)
+        if (adj_takes_u(P, nsl)) {
+            if (!rc) rc = hip_rc(hipStreamWaitEvent(st, lane->dual_done, 0), "dual wait");
+            if (!rc) rc = launch_adj_u(P, nsl, st);
+            continue;
+        }
         if (!rc) rc = launch_adj(P, nsl, false, st, true);
         if (!rc) rc = hip_rc(hipStreamWaitEvent(st, lane->dual_done, 0), "dual wait");
         if (!rc) rc = launch_primal_part(P, PRIMAL_U, st);

@@ -265,6 +265,10 @@ int launch_fwd(const ProbDev& P, const Geometry& g, int nslices, int mode, hipSt
 // the primal step of the iteration (primal == true); beside: the launch
 // shares the GPU with the dual step (two-stream schedule)
 int launch_adj(const ProbDev& P, int nslices, bool primal, hipStream_t st, bool beside = false);
+// Backprojection and u half of the primal step in one launch, where the bins of
+// a small stack are read directly (adj_takes_u); the dual step has to be over.
+bool adj_takes_u(const ProbDev& P, int nslices);
+int launch_adj_u(const ProbDev& P, int nslices, hipStream_t st);
 // Whether the single-problem stencil kernels stream with the non-temporal
 // hint: the stencil state (u, ubar, p, pbar, v, w, K^T lam) above
 // STREAM_HINT_MB; GRAPTOR_STREAM_HINTS = 0 or 1 forces the choice.  Per

@@ -691,7 +691,9 @@ __device__ __forceinline__ void adj_body(const ProbDev& P, const AdjItem& I, flo
 // without a tile: four to eight times the waves, no staging between barriers,
 // and 8 angles' reads in flight.  Bound by the latency of these reads; 183 x
 // 183, 90 angles 32 us by tiles, 9.8 so; 317 x 317 x 3, 71 angles 43 and 16.
-template <int K>
+// UDIM: the u half of the primal step of 2 or 3 dimensions follows for the
+// pixel (0: none).
+template <int K, int UDIM, bool TGV>
 __device__ __forceinline__ void adj_direct_body(const ProbDev& P, const AdjItem& I)
 {
     __shared__ float4 par[ADJ_THREADS];
@@ -739,17 +741,22 @@ __device__ __forceinline__ void adj_direct_body(const ProbDev& P, const AdjItem&
     if (x >= nx || y >= ny) return;
     const size_t plane = (size_t)nx * ny;
 #pragma unroll
-    for (int k = 0; k < K; ++k)
-        if (I.s0 + k <= last) P.ktl[(size_t)(I.s0 + k) * plane + (size_t)y * nx + x] = acc[k];
+    for (int k = 0; k < K; ++k) {
+        const int s = I.s0 + k;
+        if (s > last) continue;
+        const size_t i = (size_t)s * plane + (size_t)y * nx + x;
+        P.ktl[i] = acc[k];
+        if constexpr (UDIM > 0) primal_update<UDIM, TGV, PRIMAL_U>(P, i, x, y, s % P.nz, acc[k]);
+    }
 }
 
-template <int K>
+template <int K, int UDIM = 0, bool TGV = false>
 __global__ __launch_bounds__(ADJ_THREADS) void adj_direct_kernel(ProbDev P, int tiles_x,
                                                                  int ntiles)
 {
     const int work = xcd_work_id(blockIdx.x, gridDim.x), tile = work % ntiles;
-    adj_direct_body<K>(P, AdjItem{0, tile % tiles_x * ADJ_TX, tile / tiles_x * 4,
-                                  (work / ntiles) * K});
+    adj_direct_body<K, UDIM, TGV>(P, AdjItem{0, tile % tiles_x * ADJ_TX, tile / tiles_x * 4,
+                                              (work / ntiles) * K});
 }
 
 template <int K, bool PRIMAL, int DIM, bool TGV, int MAXR>
@@ -1044,14 +1051,59 @@ static int adj_single_k(const ProbDev& Pin, int nslices, bool primal, hipStream_
 }
 
 template <int K>
-static int adj_direct_k(const ProbDev& P, int nslices, hipStream_t st)
+static int adj_direct_k(const ProbDev& P, int nslices, bool u_half, hipStream_t st)
 {
     const int tiles_x = (P.nx + ADJ_TX - 1) / ADJ_TX, ntiles = tiles_x * ((P.ny + 3) / 4);
-    const int groups = (nslices + K - 1) / K;
-    hipLaunchKernelGGL((adj_direct_kernel<K>), dim3((unsigned)(groups * ntiles)),
-                       dim3(ADJ_THREADS), 0, st, P, tiles_x, ntiles);
+    const dim3 grd((unsigned)((nslices + K - 1) / K * ntiles)), blk(ADJ_THREADS);
+#define GR_AD(...) \
+    hipLaunchKernelGGL((adj_direct_kernel<__VA_ARGS__>), grd, blk, 0, st, P, tiles_x, ntiles)
+    if constexpr (K == 1) {
+        if (u_half && P.dim == 2) { if (P.tgv) GR_AD(1, 2, true); else GR_AD(1, 2, false); }
+        else if (u_half) { if (P.tgv) GR_AD(1, 3, true); else GR_AD(1, 3, false); }
+        else GR_AD(1);
+    } else {
+        GR_AD(K);
+    }
+#undef GR_AD
     GR_LAUNCH_CHECK("adj_direct_kernel");
     return GR_OK;
+}
+
+// Where the tiles would not give every CU a work-group, a small stack is
+// read directly, in at most 6144 waves and with as few slices per wave as
+// that allows.  One call, 60 angles, us with 1 / 2 / 4 slices a wave
+// against tiles: 64 x 64 x 1 12.5 to 20, x 64 12.6 / 12.2 / 12.4 to 32;
+// 183 x 183 x 3 12 to 22, x 16 21 / 19 / 19 to 32, x 64 (288 work-groups)
+// 64 / 49 / 43 to 37; 256 x 256 x 24 (192) 46 / 36 / 32 to 33, x 32 (256)
+// 58 / 45 / 39 to 33; 512 x 512 x 1 12 to 33, x 4 31 / 25 / 24 to 35.
+// Whole iterations: 183 x 183 x 16 71 to 78, 512 x 512 x 4 94 to 109, but
+// 64 x 64 x 256 (256 work-groups) 89 to 86, 256 x 256 x 24 (384) 116 to 108.
+// Bins narrower than a pixel stay with the tiles at every size.
+// Returns the slices per wave, 0: by tiles.
+static int adj_direct_slices(const ProbDev& P, int nslices, bool wide)
+{
+    if (P.narrow_bins || P.adj_tile_y < 4 || P.adj_tile_y % 4 != 0) return 0;
+    const long long cols = (P.nx + ADJ_TX - 1) / ADJ_TX, rows = cols * P.ny;
+    const long long tiles = cols * ((P.ny + P.adj_tile_y - 1) / P.adj_tile_y);
+    const int K = wide ? 8 : slice_group(nslices);
+    if (tiles * ((nslices + K - 1) / K) >= 256) return 0;
+    for (int d = 1; d <= 4; d *= 2)
+        if (rows * ((nslices + d - 1) / d) <= 6144) return d;
+    return 0;
+}
+
+// With one slice per wave: iterations of 64 x 64 x 1 48 to 41 us, 183 x 183 x 4
+// 55 to 48, 256 x 256 x 4 61 to 51, 512 x 512 x 1 79 to 76 (a launch and a gap
+// less).  With more, the reads of an angle are no longer issued ahead (41
+// registers instead of 89): 512 x 512 x 4 94 to 127 us.
+bool adj_takes_u(const ProbDev& P, int nslices)
+{
+    return nslices > 0 && adj_direct_slices(P, nslices, false) == 1;
+}
+
+int launch_adj_u(const ProbDev& P, int nslices, hipStream_t st)
+{
+    return adj_direct_k<1>(P, nslices, true, st);
 }
 
 int launch_adj(const ProbDev& P, int nslices, bool primal, hipStream_t st, bool beside)
@@ -1064,26 +1116,10 @@ int launch_adj(const ProbDev& P, int nslices, bool primal, hipStream_t st, bool 
     // slices, 90 angles), nor beside the dual step (0.7874 against 0.7860 ms
     // per two-stream iteration).
     const bool wide = nslices >= 8 && !primal && !beside && P.adj_tile_y <= 16;
-    // Where the tiles would not give every CU a work-group, a small stack is
-    // read directly, in at most 6144 waves and with as few slices per wave as
-    // that allows.  One call, 60 angles, us with 1 / 2 / 4 slices a wave
-    // against tiles: 64 x 64 x 1 12.5 to 20, x 64 12.6 / 12.2 / 12.4 to 32;
-    // 183 x 183 x 3 12 to 22, x 16 21 / 19 / 19 to 32, x 64 (288 work-groups)
-    // 64 / 49 / 43 to 37; 256 x 256 x 24 (192) 46 / 36 / 32 to 33, x 32 (256)
-    // 58 / 45 / 39 to 33; 512 x 512 x 1 12 to 33, x 4 31 / 25 / 24 to 35.
-    // Whole iterations: 183 x 183 x 16 71 to 78, 512 x 512 x 4 94 to 109, but
-    // 64 x 64 x 256 (256 work-groups) 89 to 86, 256 x 256 x 24 (384) 116 to 108.
-    // Bins narrower than a pixel stay with the tiles at every size.
-    if (!primal && !P.narrow_bins && P.adj_tile_y >= 4 && P.adj_tile_y % 4 == 0) {
-        const long long cols = (P.nx + ADJ_TX - 1) / ADJ_TX, rows = cols * P.ny;
-        const long long tiles = cols * ((P.ny + P.adj_tile_y - 1) / P.adj_tile_y);
-        const int K = wide ? 8 : slice_group(nslices);
-        if (tiles * ((nslices + K - 1) / K) < 256) {
-            if (rows * nslices <= 6144) return adj_direct_k<1>(P, nslices, st);
-            if (rows * ((nslices + 1) / 2) <= 6144) return adj_direct_k<2>(P, nslices, st);
-            if (rows * ((nslices + 3) / 4) <= 6144) return adj_direct_k<4>(P, nslices, st);
-        }
-    }
+    const int direct = primal ? 0 : adj_direct_slices(P, nslices, wide);
+    if (direct == 4) return adj_direct_k<4>(P, nslices, false, st);
+    if (direct == 2) return adj_direct_k<2>(P, nslices, false, st);
+    if (direct == 1) return adj_direct_k<1>(P, nslices, false, st);
     if (wide) return adj_single_k<8>(P, nslices, primal, st);
     switch (slice_group(nslices)) {
     case 4: return adj_single_k<4>(P, nslices, primal, st);
