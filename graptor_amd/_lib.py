@@ -33,7 +33,7 @@ EXPORTS = (
     "gr_tgv_energy", "gr_tgv_profile", "gr_plan_create", "gr_plan_destroy",
     "gr_plan_iterate", "gr_plan_iterate_graph", "gr_plan_profile", "gr_plan_retune",
     "gr_cnn_conv_fwd", "gr_cnn_conv_wgrad", "gr_cnn_bias_grad", "gr_cnn_weight_flip",
-    "gr_cnn_relu_bwd", "gr_cnn_pool", "gr_cnn_upsample", "gr_cnn_pack_bf16", "gr_cnn_mse_grad",
+    "gr_cnn_relu_bwd", "gr_cnn_relu_bias_grad", "gr_cnn_pool", "gr_cnn_upsample", "gr_cnn_pack_bf16", "gr_cnn_mse_grad",
     "gr_cnn_adam", "gr_tgv_dual_step", "gr_tgv_primal_step", "gr_csr_apply", "gr_prox",
     "gr_sumsq_f64", "gr_tgv_pack_halos", "gr_tgv_energy_noalloc",
 )
@@ -122,6 +122,7 @@ def load(path: str | None = None):
             "gr_cnn_bias_grad": ([V, I, I, S, I, V, V], I),
             "gr_cnn_weight_flip": ([V, V, I, I, I, V], I),
             "gr_cnn_relu_bwd": ([V, I, I, V, I, I, S, I, V], I),
+            "gr_cnn_relu_bias_grad": ([V, I, I, V, I, I, S, I, V, V], I),
             "gr_cnn_pool": ([V, I, I, V, I, I, I, I, I, I, I, I, V], I),
             "gr_cnn_upsample": ([V, I, I, V, I, I, I, I, I, I, I, V], I),
             "gr_cnn_pack_bf16": ([V, I, V, I, I, S, F, V], I),

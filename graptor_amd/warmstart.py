@@ -267,14 +267,17 @@ class UNet:
 
         def layer_back(name, xin: View, dy: View, yout: View, dx: View | None):
             l = L[name]
+            db = self.g.data_ptr() + 4 * l.b_off
             if l.relu:
-                _lib.check(lib.gr_cnn_relu_bwd(dy.ptr, dy.ld, dy.c0, yout.ptr, yout.ld, yout.c0,
-                                               dy.npix(), l.cout, st), "relu_bwd")
+                _lib.check(lib.gr_cnn_relu_bias_grad(dy.ptr, dy.ld, dy.c0, yout.ptr, yout.ld,
+                                                     yout.c0, dy.npix(), l.cout, db, st),
+                           "relu_bias_grad")
+            else:
+                _lib.check(lib.gr_cnn_bias_grad(dy.ptr, dy.ld, dy.c0, dy.npix(), l.cout, db, st),
+                           "bias_grad")
             _lib.check(lib.gr_cnn_conv_wgrad(xin.ptr, xin.ld, xin.c0, dy.ptr, dy.ld, dy.c0,
                                              self.g.data_ptr() + 4 * l.w_off, n, xin.h, xin.w,
                                              l.cin, l.cout, l.taps, xin.h, st), "wgrad")
-            _lib.check(lib.gr_cnn_bias_grad(dy.ptr, dy.ld, dy.c0, dy.npix(), l.cout,
-                                            self.g.data_ptr() + 4 * l.b_off, st), "bias_grad")
             if dx is not None:
                 wf = self.wflip[name]
                 _lib.check(lib.gr_cnn_weight_flip(self.pb.data_ptr() + 2 * l.w_off,

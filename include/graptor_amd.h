@@ -293,6 +293,9 @@ int gr_cnn_weight_flip(const void *w, void *wt, int cin, int cout, int taps, voi
 /* dy *= (y > 0), in place */
 int gr_cnn_relu_bwd(void *dy, int ldd, int cd0, const void *y, int ldy, int cy0, size_t npix,
                     int c, void *stream);
+/* both at once: dy *= (y > 0), then db[co] += sum of the masked dy */
+int gr_cnn_relu_bias_grad(void *dy, int ldd, int cd0, const void *y, int ldy, int cy0,
+                          size_t npix, int cout, float *db, void *stream);
 /* backward == 0: y = 2x2 average pool of x (H, W of x).  backward != 0: y (fine,
  * H x W) = 1/4 x (coarse) broadcast, added to y when accumulate != 0. */
 int gr_cnn_pool(const void *x, int ldx, int cx0, void *y, int ldy, int cy0, int n, int H, int W,
