@@ -97,7 +97,7 @@ def load(path: str | None = None):
             "gr_geometry_get_tuning": ([V, PI, PI], I),
             "gr_geometry_set_fusion": ([V, I], I),
             "gr_radon": ([V, V, V, I, V], I),
-            "gr_radon_scratch": ([V, V, V, I, V, V], I),
+            "gr_radon_scratch": ([V, V, V, I, V, I, V], I),
             "gr_radon_scratch_floats": ([V, I], ctypes.c_size_t),
             "gr_radon_ad": ([V, V, V, I, V], I),
             "gr_normest": ([V, V, I, I, D, PD, V], I),

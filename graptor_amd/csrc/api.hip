@@ -82,6 +82,8 @@ struct ShearTables {
 bool make_shear(const std::vector<FwdAngle>& fa, int nd, int nlines, ShearTables& T)
 {
     const int na = (int)fa.size();
+    // an item per bin at least, and 16 waves hold 1024
+    if (nd + 2 > FWD_LINE_ITEMS) return false;
     // |mcand| <= 1: three bins per item; >= FWD_SHEAR_MIN: at most
     // FWD_BIN_ITEMS items per bin, and not many more items than bins.  An
     // offset beyond +-1e6 bins could overflow an item's line index.
@@ -97,17 +99,16 @@ bool make_shear(const std::vector<FwdAngle>& fa, int nd, int nlines, ShearTables
     for (int a = 0; a < na; ++a) {
         // products of these floats and a line's or candidate's number are exact
         const double ms = fa[a].mstep, mc = fa[a].mcand, off = fa[a].off, inv = 1.0 / mc;
-        auto bin = [&](long long j) { return nearest((double)j * mc + off); };
+        auto at = [&](long long j) { return (double)j * mc + off; };
         // items whose nearest bin is -1 .. nd
-        long long j0 = (long long)std::floor(((mc > 0 ? -1.5 : nd + 0.5) - off) / mc) - 2;
-        auto in = [&](long long j) { return bin(j) >= -1 && bin(j) <= nd; };
-        while (!in(j0)) ++j0;
-        const size_t first = T.lines.size();
-        T.line0.push_back((int)first);
+        long long j = (long long)std::floor(((mc > 0 ? -1.5 : nd + 0.5) - off) / mc) - 2;
+        long long b = nearest(at(j));
+        while (b < -1 || b > nd) b = nearest(at(++j));
+        T.line0.push_back((int)T.lines.size());
         m.clear();
-        for (long long j = j0; in(j); ++j) {
-            m.push_back((int)bin(j));
-            T.lines.push_back(FwdLine{(int)j, (float)((double)j * mc + off - (double)m.back())});
+        for (; b >= -1 && b <= nd; b = nearest(at(++j))) {
+            m.push_back((int)b);
+            T.lines.push_back(FwdLine{(int)j, (float)(at(j) - (double)b)});
         }
         const size_t b0 = T.bins.size();
         T.bins.resize(b0 + nd, FwdBin{0, 0});
@@ -823,43 +824,35 @@ int gr_geometry_create(const float* ofs, int na, int nx, int ny, int nd, gr_geom
     }
     g.tab_off[4] = (int)g.chunks_host.size();
     ShearTables sh;
-    const bool sheared = make_shear(fa, nd, std::max(nx, ny) + SHEAR_BLOCK, sh);
-    hipError_t e = hipMalloc(&g.ofs_dev, sizeof(float) * 4 * na);
-    if (e == hipSuccess) e = hipMalloc(&g.fwd_dev, sizeof(FwdAngle) * na);
-    if (e == hipSuccess) e = hipMalloc(&g.chunks_dev, sizeof(FwdChunk) * g.chunks_host.size());
-    if (e == hipSuccess)
-        e = hipMemcpy(g.ofs_dev, ofs, sizeof(float) * 4 * na, hipMemcpyHostToDevice);
-    if (e == hipSuccess)
-        e = hipMemcpy(g.fwd_dev, fa.data(), sizeof(FwdAngle) * na, hipMemcpyHostToDevice);
-    if (e == hipSuccess)
-        e = hipMemcpy(g.chunks_dev, g.chunks_host.data(), sizeof(FwdChunk) * g.chunks_host.size(),
-                      hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-        int rc = hip_status(e, "geometry_create");
+    const bool sheared = (long long)nx * ny >= FWD_LINE_PIXELS &&
+                         make_shear(fa, nd, std::max(nx, ny) + SHEAR_BLOCK, sh);
+    // one allocation, owned by ofs_dev, and one copy for all tables
+    std::vector<char> all;
+    auto put = [&](const void* p, size_t n) {
+        const size_t at = all.size();
+        all.resize((at + n + 63) / 64 * 64);
+        std::memcpy(all.data() + at, p, n);
+        return at;
+    };
+    auto puts = [&](const auto& v) { return v.empty() ? 0 : put(v.data(), sizeof(v[0]) * v.size()); };
+    put(ofs, sizeof(float) * 4 * na);
+    const size_t fwd = puts(fa), chunks = puts(g.chunks_host);
+    const size_t shear = sheared ? puts(sh.shear) : 0, lines = sheared ? puts(sh.lines) : 0;
+    const size_t line0 = sheared ? puts(sh.line0) : 0, bins = sheared ? puts(sh.bins) : 0;
+    char* dev = nullptr;
+    const int rc = upload(all, &dev);
+    g.ofs_dev = reinterpret_cast<float*>(dev);
+    if (rc) {
         gr_geometry_destroy(gg);
         return rc;
     }
+    g.fwd_dev = reinterpret_cast<FwdAngle*>(dev + fwd);
+    g.chunks_dev = reinterpret_cast<FwdChunk*>(dev + chunks);
     if (sheared) {
         g.shear_stride = std::max(nx, ny) + SHEAR_BLOCK;
         for (int a = 0; a < na; ++a)
             g.shear_waves = std::max(g.shear_waves, (sh.line0[a + 1] - sh.line0[a] + 63) / 64);
-        // one allocation and one copy for the four tables
-        std::vector<char> all;
-        auto put = [&](const auto& v) {
-            const size_t at = all.size(), n = sizeof(v[0]) * v.size();
-            all.resize((at + n + 63) / 64 * 64);
-            std::memcpy(all.data() + at, v.data(), n);
-            return at;
-        };
-        put(sh.shear);
-        const size_t lines = put(sh.lines), line0 = put(sh.line0), bins = put(sh.bins);
-        char* dev = nullptr;
-        int rc = upload(all, &dev);
-        g.shear_dev = reinterpret_cast<Shear*>(dev);
-        if (rc) {
-            gr_geometry_destroy(gg);
-            return rc;
-        }
+        g.shear_dev = reinterpret_cast<Shear*>(dev + shear);
         g.lines_dev = reinterpret_cast<FwdLine*>(dev + lines);
         g.line0_dev = reinterpret_cast<int*>(dev + line0);
         g.bins_dev = reinterpret_cast<FwdBin*>(dev + bins);
@@ -873,9 +866,6 @@ int gr_geometry_destroy(gr_geometry* gg)
     if (!gg) return GR_OK;
     Geometry& g = gg->g;
     if (g.ofs_dev) (void)hipFree(g.ofs_dev);
-    if (g.fwd_dev) (void)hipFree(g.fwd_dev);
-    if (g.chunks_dev) (void)hipFree(g.chunks_dev);
-    if (g.shear_dev) (void)hipFree(g.shear_dev);
     delete gg;
     return GR_OK;
 }
@@ -937,9 +927,9 @@ size_t gr_radon_scratch_floats(const gr_geometry* gg, int nslices)
 }
 
 int gr_radon_scratch(const gr_geometry* gg, float* sino, const float* img, int nslices,
-                     float* scratch, void* stream)
+                     float* scratch, int of_slices, void* stream)
 {
-    if (!gg || !sino || !img || nslices < 0 || !scratch || scratch == img) {
+    if (!gg || !sino || !img || nslices < 0 || !scratch || scratch == img || of_slices < 0) {
         set_error("radon_scratch: invalid arguments");
         return GR_ERR_INVALID;
     }
@@ -948,7 +938,11 @@ int gr_radon_scratch(const gr_geometry* gg, float* sino, const float* img, int n
     P.ubar = const_cast<float*>(img);
     P.ku = sino;
     P.ktl = scratch;
-    return launch_fwd(P, gg->g, nslices, FWD_WRITE | FWD_SCRATCH | FWD_ALONE, stream_of(stream));
+    int mode = FWD_WRITE | FWD_SCRATCH | FWD_ALONE;
+    if (of_slices > 0)  // the way an iteration of the whole goes
+        mode = fwd_by_lines(standalone(gg, of_slices), gg->g) ? FWD_WRITE | FWD_SCRATCH | FWD_LINES
+                                                              : FWD_WRITE;
+    return launch_fwd(P, gg->g, nslices, mode, stream_of(stream));
 }
 
 int gr_radon_ad(const gr_geometry* gg, float* img, const float* sino, int nslices, void* stream)

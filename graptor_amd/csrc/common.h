@@ -110,10 +110,13 @@ struct DualItem { int prob, x0, y0, z; };
 
 constexpr int SHEAR_BLOCK = 8;       // lines per table read
 constexpr double FWD_SHEAR_MIN = 0.7;
+constexpr int FWD_LINE_ITEMS = 1024;  // items of an angle: 16 waves
+constexpr long long FWD_LINE_PIXELS = 6400;  // smaller slices are never projected by lines
 
 // Device-side geometry (owned by gr_geometry).
 struct Geometry {
     int nx, ny, nd, na;
+    // device tables, one allocation owned by ofs_dev
     float* ofs_dev;          // na x float4 (cos, sin, off, 1/cos) as given
     FwdAngle* fwd_dev;       // na, sorted by class
     FwdChunk* chunks_dev;    // four chunk tables back to back
@@ -121,7 +124,7 @@ struct Geometry {
                              // built for 8, 4, 2, 1 items per thread
     std::vector<FwdChunk> chunks_host;
     // sheared projection (every |mcand| in [FWD_SHEAR_MIN, 1], i.e. unit
-    // detector bins); otherwise null.  One allocation, owned by shear_dev
+    // detector bins); otherwise null
     Shear* shear_dev;        // na x shear_stride
     FwdLine* lines_dev;
     int* line0_dev;          // na + 1
@@ -142,10 +145,11 @@ struct Geometry {
 // the dual step may size it for its grid.
 // FWD_SCRATCH: P.ktl (as large as the image) may be overwritten: inside an
 // iteration, where the backprojection fills it afterwards, or because the
-// caller says so.  FWD_ALONE: no dual step beside the launch.
+// caller says so.  FWD_ALONE: no dual step beside the launch.  FWD_LINES: by
+// lines, whatever fwd_by_lines says of this stack.
 enum {
     FWD_WRITE = 1, FWD_KL = 2, FWD_L2 = 4, FWD_PROX = 8, FWD_BESIDE = 16, FWD_AUTOBAND = 32,
-    FWD_SCRATCH = 64, FWD_ALONE = 128
+    FWD_SCRATCH = 64, FWD_ALONE = 128, FWD_LINES = 256
 };
 
 // Map hardware block order (dealt round-robin over the 8 XCDs) to a work

@@ -143,7 +143,7 @@ def radon(sino, img, r_struct, wait_for=None):
     tmp = _radon_scratch(lib.gr_radon_scratch_floats(g.handle, ns_i), img.device)
     if tmp is not None:
         _lib.check(lib.gr_radon_scratch(g.handle, sv.data_ptr(), imv.data_ptr(), ns_i,
-                                        tmp.data_ptr(), _stream_ptr(img)), "radon")
+                                        tmp.data_ptr(), 0, _stream_ptr(img)), "radon")
         return
     _lib.check(lib.gr_radon(g.handle, sv.data_ptr(), imv.data_ptr(), ns_i,
                             _stream_ptr(img)), "radon")

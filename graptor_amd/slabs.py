@@ -26,7 +26,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .projector import RadonGeometry, radon, radon_ad
+from .projector import RadonGeometry, radon_ad
 from .solver import TgvProblem
 
 class SlabSolve:
@@ -47,7 +47,7 @@ class SlabSolve:
                                  device=device)
                       for z0, z1 in zip(bounds[:-1], bounds[1:])]
         self.bounds = [(int(a), int(b)) for a, b in zip(bounds[:-1], bounds[1:])]
-        self.geometry = geometry
+        self.geometry, self.Nz = geometry, int(Nz)
         self.tgv = regularisation.upper() == "TGV"
         self.halos = []
         for s, p in enumerate(self.slabs):
@@ -105,7 +105,10 @@ class SlabSolve:
                                                 ctypes.byref(p.state), st), "dual_step")
             for p in self.slabs:
                 S = p.C * p.Nz
-                radon(p.ku.view(S, p.na, p.nd), p.ubar.view(S, p.ny, p.nx), self.geometry)
+                # K^T lam is written next: scratch of the projection until then
+                _lib.check(lib.gr_radon_scratch(self.geometry.handle, p.ku.data_ptr(),
+                                                p.ubar.data_ptr(), S, p.ktl.data_ptr(),
+                                                p.C * self.Nz, p._stream()), "radon")
                 _lib.check(lib.gr_prox(_lib.DISCREPANCY[p.discrepancy], float(p.params.sigma_p),
                                        p.mfac.data_ptr(), p.C, p.Nz * p.na * p.nd,
                                        p.ku.data_ptr(), p.f.data_ptr(), p.lam.data_ptr(),

@@ -201,7 +201,7 @@ class SubsampledProblem:
                                 (self.g1, k1_fine, img[C0:], scratch[C0:])):
             if part.shape[0]:
                 _lib.check(lib.gr_radon_scratch(g.handle, k.data_ptr(), part.data_ptr(),
-                                                part.shape[0] * nz, tmp.data_ptr(), st), "radon")
+                                                part.shape[0] * nz, tmp.data_ptr(), 0, st), "radon")
         self.S.apply(k1_fine, k1, self.na1, C1, self._stream())
 
     def _adjoint(self, l0, l1, l1_fine, out):

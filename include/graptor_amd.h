@@ -71,10 +71,12 @@ int gr_radon(const gr_geometry *g, float *sino, const float *img, int nslices,
              void *stream);
 /* The same with a scratch array of at least gr_radon_scratch_floats floats, apart
  * from img, which is overwritten: small stacks are then projected by lines, two
- * to seven times as fast.  0 floats: gr_radon does as well. */
+ * to seven times as fast.  0 floats: gr_radon does as well.  of_slices > 0: the
+ * slices are part of a stack of so many and get the bits that an iteration of
+ * the whole stack gives them (scratch: as large as img). */
 size_t gr_radon_scratch_floats(const gr_geometry *g, int nslices);
 int gr_radon_scratch(const gr_geometry *g, float *sino, const float *img, int nslices,
-                     float *scratch, void *stream);
+                     float *scratch, int of_slices, void *stream);
 
 /* Replaces radon_ad() 2D:559-565 / 3D:1002-1008 (kernel 2D:436-462):
  * img[s] = R^T sino[s]. */
@@ -142,7 +144,7 @@ typedef struct gr_tgv_state {
 
 /* Runs n_iter iterations of the loop 2D:767-799 / 3D:1194-1221 on `stream`:
  * dual step with the coupled projections; forward projection fused with the
- * KL/L2 prox; backprojection; primal step fused with the extrapolation
+ * KL/L2 prox (which may use st->ktl as scratch); backprojection, which fills it; primal step fused with the extrapolation
  * (inside the backprojection kernel when the geometry's fusion is on, in
  * which case st->ktl may be NULL).  With ku_on_last,
  * the last iteration also stores R(ubar) into ku, the sinogram the reference

@@ -81,4 +81,23 @@ def test_projection_with_scratch(case):
     n = _lib.load().gr_radon_scratch_floats(g.handle, S)
     assert n in (0, S * nx * ny)
     assert _lib.load().gr_radon_scratch(g.handle, sino.data_ptr(), img.data_ptr(), S,
-                                        img.data_ptr(), None) == _lib.GR_ERR_INVALID
+                                        img.data_ptr(), 0, None) == _lib.GR_ERR_INVALID
+
+
+@pytest.mark.parametrize("C,nz,reg", [(3, 8, "TGV"), (1, 33, "TV"), (4, 12, "TGV")])
+def test_slabs_of_a_small_volume_give_its_bits(C, nz, reg):
+    """Whole: by lines (24 slices, with the u half of the primal step behind the
+    backprojection; 33 slices) and by the gather (48 are too many for 96 x 96)."""
+    from graptor_amd.projector import RadonGeometry
+    from graptor_amd.slabs import SlabSolve
+    from graptor_amd.solver import TgvProblem
+    print(f"slabs of {C} x {nz}", flush=True)
+    g = RadonGeometry((96, 96), angles_deg(-70, 70, 40), n_detectors=96)
+    f = np.random.default_rng(nz).random((C, nz, 40, 96)).astype(np.float32)
+    kw = dict(coupling="frobenius", discrepancy="KL", regularisation=reg, L=40.0)
+    whole = TgvProblem(f, g, (4.0, 1.0), [1.0] * C, dim=3, **kw)
+    parts = SlabSolve(f, g, (4.0, 1.0), [1.0] * C, 3, **kw)
+    whole.iterate(6)
+    parts.iterate(6)
+    for name in ("u", "v", "lam", "ktl"):
+        assert torch.equal(getattr(whole, name), parts.gather(name)), name
