@@ -241,10 +241,10 @@ __global__ __launch_bounds__(256) void conv_tile_kernel(
 // U-Net of 32 images of 256 x 256, all 3x3 layers: 2366 us by tiles, 1440 so
 // (32 output channels at 256 x 256: 212 to 139 us a layer; 64 at 128 x 128:
 // 142 to 104; 128 at 64 x 64 and 256 at 32 x 32: 161 to 78); 700 GFLOP, 580 us
-// at the rate of a large product.  Two output tiles per wave (TN = 2) need
-// spills at 4 rows: 64 x 64 85 instead of 78 us.  What bounds it now: one or
-// two work-groups per CU, whose staging is not all hidden, and at 256 x 256 memory
-// (1.3 GB, 277 us at 4.6 TB/s, of 556).
+// at the rate of a large product.  Two output tiles per wave (TN = 2) spill at
+// 4 rows: the whole inference 1745 us with them at 64 x 64, 1886 at 32 x 32, 1651
+// with one.  What bounds it now: one or two work-groups per CU, whose staging is
+// not all hidden, and at 256 x 256 memory (1.3 GB, 277 us at 4.6 TB/s, of 556).
 // ---------------------------------------------------------------------------
 template <int WAVES_M_, int TM_, int TN_, int KC_>
 struct ConvRows {

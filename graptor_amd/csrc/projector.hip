@@ -117,7 +117,7 @@ __device__ __forceinline__ void fwd_epilogue(const ProbDev& P, int mode, int s0,
 // of lines in LDS behind barriers and finds each ray's candidates from the
 // ray, 5 operations and a read for each of 3 candidates; with a work-group or
 // less per CU its time is that chain's latency.  Here a line costs an item
-// one read and 3 operations, in flight 8 at a time.  Bound by the L1's rate
+// one read and 3 operations a slice and 5 for the weights, 8 lines in flight.  Bound by the L1's rate
 // (about 8 cycles a wave's read) and, for single slices, by latency; two
 // halves give single slices twice the waves (317 x 317 x 3, 71 angles, 10
 // iterations: 1000 us with one wave, 898 with two; 183 x 183: 680, 630).
