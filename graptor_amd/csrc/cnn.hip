@@ -13,6 +13,7 @@
 //   B[k][n]: lane holds n = l % 32, k = 8h .. 8h+7
 //   D[m][n]: lane holds n = l % 32, rows m = 8(r/4) + 4h + r%4, r = 0..15
 #include "common.h"
+#include "wgrad_walk.h"
 
 #include <hip/hip_bf16.h>
 
@@ -463,16 +464,13 @@ __global__ __launch_bounds__(256, 2) void conv_wgrad_kernel(
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = lane >> 5, l32 = lane & 31;
     const int co_blocks = (cout + 31) / 32, ci_blocks = (cin + 31) / 32;
-    const int segs = (W + SEG - 1) / SEG, row_chunks = (H + rows - 1) / rows;
     int b = xcd_work_id(blockIdx.x, gridDim.x);
     const int cob = b % co_blocks * 32;
     b /= co_blocks;
     const int cib = b % ci_blocks * 32;
     b /= ci_blocks;
-    const int unit = 4 * b + wave;  // (image, segment, chunk of rows)
-    const int img = unit / (segs * row_chunks), us = unit - img * segs * row_chunks;
-    const int x0 = us / row_chunks * SEG, r0 = us % row_chunks * rows;
-    const int nrows = img < n ? min(rows, H - r0) : 0;
+    const WgradUnit U = wgrad_unit<SEG>(4 * b + wave, n, H, W, rows);
+    const int img = U.img, x0 = U.x0, r0 = U.r0, nrows = U.nrows;
 
     // staging role: 8 pixels (block j) x 8 channels (group g) of dy or of x
     const int kind = lane / (SEG / 2), sub = lane % (SEG / 2), g = sub & 3, j = sub >> 2;
@@ -485,8 +483,8 @@ __global__ __launch_bounds__(256, 2) void conv_wgrad_kernel(
     uint16_t* my = lds + wave * WAVE;
     u32x4 v[8], ve[2];  // ve: the two pixels of x after the last block
     auto load = [&](int t) {
-        const int row = r0 + t + (is_x ? HALO : 0);
-        const bool ok = ch_ok && row >= 0 && row < H && t < nrows && (is_x || t >= 0);
+        const int row = wgrad_row(r0, t, is_x, HALO);
+        const bool ok = ch_ok && wgrad_row_ok(row, t, nrows, H, is_x);
         const uint16_t* at = src + (size_t)(img * H + row) * W * ld;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -532,9 +530,10 @@ __global__ __launch_bounds__(256, 2) void conv_wgrad_kernel(
         for (int r = 0; r < 16; ++r) acc[d][r] = 0.f;
 
     // row t of dy meets rows t - 1, t, t + 1 of x, stored by steps t - 2, t - 1, t
+    const int first = wgrad_first(nrows, HALO);
     int slot = 0;
-    if (nrows > 0) load(-2 * HALO);
-    for (int t = -2 * HALO; t < nrows; ++t) {
+    if (first < nrows) load(first);
+    for (int t = first; t < nrows; ++t) {
         // the wave's own LDS operations complete in order; the compiler must
         // keep them in order too
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -1016,18 +1015,10 @@ static void conv_wgrad_launch(const uint16_t* x, int ldx, int cx0, const uint16_
 {
     const long long tiles = (long long)((cout + 31) / 32) * ((cin + 31) / 32);
     const long long columns = (long long)n * ((W + SEG - 1) / SEG);
-    // Rows per wave: long walks read x once and add fewer partial sums, but
-    // every CU should have work.  One work-group per CU, one and a half where
-    // that leaves long walks.  Training steps of n images of 256 x 256 with 256
-    // / 384 / 512 work-groups: n = 2 1162 / 1255 / 1292 us, n = 8 2003 / 1983 /
-    // 2095, n = 16 3215 / 3141 / 3215; with 128, n = 16 3451.
-    long long rows = columns * H * tiles / (4 * 256);
-    if (rows >= 12) rows = rows * 2 / 3;
-    rows = std::max<long long>(1, std::min<long long>(H, rows));
+    const int rows = wgrad_rows(columns, H, tiles);
     const long long units = columns * ((H + rows - 1) / rows);
     hipLaunchKernelGGL((conv_wgrad_kernel<TAPS, SEG>), dim3((unsigned)(tiles * ((units + 3) / 4))),
-                       dim3(256), 0, st, x, ldx, cx0, dy, ldd, cd0, dw, n, H, W, cin, cout,
-                       (int)rows);
+                       dim3(256), 0, st, x, ldx, cx0, dy, ldd, cd0, dw, n, H, W, cin, cout, rows);
 }
 
 extern "C" {
