@@ -5,7 +5,9 @@ of the backprojection on scratch copies of the problems' state (so the real
 iterates are untouched), through the batch plan's per-phase HIP-event
 profile, and applies the fastest shapes to the geometries.  The forward band
 only affects the forward phase and the tile height only the backprojection
-phase, so the two are tuned independently.
+phase, so the two are tuned independently.  Problems whose iterations project
+by lines have no band: they are left out of its choice, and their geometries
+keep the automatic one (which larger stacks and energies on them use).
 """
 from __future__ import annotations
 
@@ -35,6 +37,11 @@ def _lds_ok(problem, band):
     return band * pitch * K * 4 <= LDS_LIMIT
 
 
+def _gathered(problems):
+    """Problems whose forward phase has a band."""
+    return [p for p in problems if not p.geometry.iterates_by_lines(p.C * p.Nz)]
+
+
 def signature(problems):
     return ";".join(f"{p.dim}:{p.C}x{p.Nz}x{p.ny}x{p.nx}:{p.na}" for p in problems)
 
@@ -42,7 +49,7 @@ def signature(problems):
 def autotune(problems, iters=3, plan=None, cache=None):
     """Tune tile shapes for ``problems`` (list of TgvProblem sharing nothing
     but the device).  Returns {"fwd_band": b, "adj_tile_y": t, "ms": {...}}
-    and leaves every geometry set to the winner.  ``plan`` (a BatchPlan over
+    (b = 0: no problem has a band) and leaves every geometry set to the winner.  ``plan`` (a BatchPlan over
     the same problems) is retuned as well.  With ``cache`` (a JSON path) a
     previous result for the same signature is reused."""
     sig = signature(problems)
@@ -58,11 +65,12 @@ def autotune(problems, iters=3, plan=None, cache=None):
     geoms = {id(p.geometry): p.geometry for p in problems}
     fwd_ms, adj_ms = {}, {}
     splan.profile(1)  # warm-up
-    for band in FWD_BANDS:
-        if not all(_lds_ok(p, band) for p in problems):
+    gathered = _gathered(problems)
+    for band in FWD_BANDS if gathered else ():
+        if not all(_lds_ok(p, band) for p in gathered):
             continue
-        for g in geoms.values():
-            g.set_tuning(fwd_band=band, adj_tile_y=16)
+        for p in gathered:
+            p.geometry.set_tuning(fwd_band=band, adj_tile_y=16)
         splan.retune()
         fwd_ms[band] = splan.profile(iters)[1] / iters
     # no candidate fits (very wide images): the forward band stays as it is
@@ -70,7 +78,7 @@ def autotune(problems, iters=3, plan=None, cache=None):
     best_band = min(fwd_ms, key=fwd_ms.get) if fwd_ms else 0
     for tile in ADJ_TILES:
         for g in geoms.values():
-            g.set_tuning(fwd_band=best_band, adj_tile_y=tile)
+            g.set_tuning(adj_tile_y=tile)
         splan.retune()
         prof = splan.profile(iters)
         adj_ms[tile] = (prof[2] + prof[3]) / iters
@@ -94,6 +102,8 @@ def autotune(problems, iters=3, plan=None, cache=None):
 
 def _apply(problems, band, tile, plan):
     for p in problems:
-        p.geometry.set_tuning(fwd_band=band, adj_tile_y=tile)
+        p.geometry.set_tuning(adj_tile_y=tile)
+    for p in _gathered(problems):
+        p.geometry.set_tuning(fwd_band=band)
     if plan is not None:
         plan.retune()

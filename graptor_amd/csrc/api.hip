@@ -896,6 +896,14 @@ int gr_geometry_set_fusion(gr_geometry* gg, int fuse_primal)
     return GR_OK;
 }
 
+int gr_iterates_by_lines(const gr_geometry* gg, int nslices)
+{
+    if (!gg || nslices <= 0) return 0;
+    ProbDev P = standalone(gg, nslices);
+    P.fuse_primal = gg->g.fuse_primal;
+    return fwd_by_lines(P, gg->g) ? 1 : 0;
+}
+
 int gr_geometry_get_tuning(const gr_geometry* gg, int* fwd_band, int* adj_tile_y)
 {
     if (!gg) {

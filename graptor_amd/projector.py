@@ -74,6 +74,11 @@ class RadonGeometry:
                    "get_tuning")
         return a.value, b.value
 
+    def iterates_by_lines(self, nslices: int) -> bool:
+        """Whether an iteration of ``nslices`` slices projects forward by lines
+        (small stacks) instead of gathering each ray's pixels."""
+        return bool(_lib.load().gr_iterates_by_lines(self._h, int(nslices)))
+
     def __del__(self):
         h = getattr(self, "_h", None)
         if h is not None and h.value:

@@ -64,6 +64,9 @@ int gr_geometry_get_tuning(const gr_geometry *g, int *fwd_band, int *adj_tile_y)
  * stored); 0 (default): backprojection writes st->ktl and a separate
  * primal kernel reads it. */
 int gr_geometry_set_fusion(gr_geometry *g, int fuse_primal);
+/* 1 if an iteration of nslices slices projects forward by lines (small stacks;
+ * fwd_band has no part in it), 0 if it gathers each ray's pixels. */
+int gr_iterates_by_lines(const gr_geometry *g, int nslices);
 
 /* Replaces radon() 2D:544-550 / 3D:988-994 (kernel 2D:391-434):
  * sino[s][angle][bin] = R img[s][y][x] for s < nslices. */
