@@ -948,8 +948,8 @@ int gr_radon_scratch(const gr_geometry* gg, float* sino, const float* img, int n
     P.ktl = scratch;
     int mode = FWD_WRITE | FWD_SCRATCH | FWD_ALONE;
     if (of_slices > 0)  // the way an iteration of the whole goes
-        mode = fwd_by_lines(standalone(gg, of_slices), gg->g) ? FWD_WRITE | FWD_SCRATCH | FWD_LINES
-                                                              : FWD_WRITE;
+        mode = gr_iterates_by_lines(gg, of_slices) ? FWD_WRITE | FWD_SCRATCH | FWD_LINES
+                                                   : FWD_WRITE;
     return launch_fwd(P, gg->g, nslices, mode, stream_of(stream));
 }
 
