@@ -723,6 +723,12 @@ int plan_iter(gr_plan* pl, int n_iter, int ku_on_last, hipStream_t st)
     return GR_OK;
 }
 
+bool overlap(const float* a, size_t na, const float* b, size_t nb)
+{
+    const uintptr_t a0 = (uintptr_t)a, b0 = (uintptr_t)b;
+    return a0 < b0 + nb * sizeof(float) && b0 < a0 + na * sizeof(float);
+}
+
 ProbDev standalone(const gr_geometry* gg, int nslices)
 {
     const Geometry& g = gg->g;
@@ -950,6 +956,12 @@ int gr_radon_scratch(const gr_geometry* gg, float* sino, const float* img, int n
     if (of_slices > 0)  // the way an iteration of the whole goes
         mode = gr_iterates_by_lines(gg, of_slices) ? FWD_WRITE | FWD_SCRATCH | FWD_LINES
                                                    : FWD_WRITE;
+    const size_t px = (size_t)P.nx * P.ny * nslices, bins = (size_t)P.na * P.nd * nslices;
+    const bool lines = (mode & FWD_LINES) || ((mode & FWD_ALONE) && fwd_by_lines(P, gg->g, true));
+    if (lines && (overlap(scratch, px, img, px) || overlap(scratch, px, sino, bins))) {
+        set_error("radon_scratch: the scratch overlaps the image or the sinogram");
+        return GR_ERR_INVALID;
+    }
     return launch_fwd(P, gg->g, nslices, mode, stream_of(stream));
 }
 

@@ -72,8 +72,8 @@ int gr_iterates_by_lines(const gr_geometry *g, int nslices);
  * sino[s][angle][bin] = R img[s][y][x] for s < nslices. */
 int gr_radon(const gr_geometry *g, float *sino, const float *img, int nslices,
              void *stream);
-/* The same with a scratch array of at least gr_radon_scratch_floats floats, apart
- * from img, which is overwritten: small stacks are then projected by lines, two
+/* The same with a scratch array of at least gr_radon_scratch_floats floats, which
+ * is overwritten and overlaps neither img nor sino: small stacks are then projected by lines, two
  * to seven times as fast.  0 floats: gr_radon does as well.  of_slices > 0: the
  * slices are part of a stack of so many and get the bits that an iteration of
  * the whole stack gives them (scratch: as large as img). */
