@@ -4,6 +4,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <atomic>
+#include <mutex>
 #include <vector>
 
 #include "../../include/graptor_amd.h"
@@ -123,14 +125,21 @@ struct Geometry {
     int tab_off[5];          // table t = chunks [tab_off[t], tab_off[t+1]),
                              // built for 8, 4, 2, 1 items per thread
     std::vector<FwdChunk> chunks_host;
-    // sheared projection (every |mcand| in [FWD_SHEAR_MIN, 1], i.e. unit
-    // detector bins); otherwise null
-    Shear* shear_dev;        // na x shear_stride
-    FwdLine* lines_dev;
-    int* line0_dev;          // na + 1
-    FwdBin* bins_dev;        // na x nd
+    // sheared projection: waves of items of the angle with the most, or 0 where
+    // it does not apply (every |mcand| in [FWD_SHEAR_MIN, 1], i.e. unit
+    // detector bins; see shear_waves_of)
+    int shear_waves;
+    // its tables, one allocation owned by shear_dev: built by the first call
+    // that needs them (line_tables) and final once shear_ready is set
+    int device;
+    std::vector<FwdAngle> fwd_host;  // as fwd_dev
+    mutable std::mutex shear_mutex;
+    mutable std::atomic<bool> shear_ready{false};
+    mutable Shear* shear_dev = nullptr;      // na x shear_stride
+    mutable const FwdLine* lines_dev;
+    mutable const int* line0_dev;            // na + 1
+    mutable const FwdBin* bins_dev;          // na x nd
     int shear_stride;
-    int shear_waves;         // waves of items of the angle with the most
     int fwd_band;            // lines per LDS band (0: automatic)
     int adj_tile_y;          // rows per backprojection tile
     int narrow_bins;         // detector width below one pixel
@@ -247,7 +256,7 @@ __device__ __forceinline__ int stencil_block()
     return ((local / G) * 8 + xcd) * G + local % G;
 }
 
-inline void set_shear(ProbDev& P, const Geometry& g)
+inline void set_shear(ProbDev& P, const Geometry& g)  // after line_tables
 {
     P.shear = g.shear_dev; P.lines = g.lines_dev; P.line0 = g.line0_dev; P.bins = g.bins_dev;
     P.shear_stride = g.shear_stride;
@@ -305,7 +314,7 @@ int launch_fwd_line_batch(const ProbDev* probs_dev, const FwdItem* items, int ni
 int launch_transpose_batch(const ProbDev* probs_dev, const DualItem* items, int nitems,
                            hipStream_t st);
 // Whether an iteration of this problem (alone: a projection outside one)
-// projects forward by lines.
+// projects forward by lines, given the tables (set_shear).
 bool fwd_by_lines(const ProbDev& P, const Geometry& g, bool alone = false);
 int launch_adj_batch(const ProbDev* probs_dev, const AdjItem* items, int nitems, int K,
                      int dim, bool tgv, bool primal, size_t lds, hipStream_t st);

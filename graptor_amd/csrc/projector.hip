@@ -942,7 +942,7 @@ bool fwd_by_lines(const ProbDev& P, const Geometry& g, bool alone)
 {
     const long long S = (long long)P.nz * P.nch, px = (long long)P.nx * P.ny;
     const long long groups = (long long)P.na * ((S + 3) / 4);
-    if (!g.shear_dev || 64 * g.shear_waves > FWD_LINE_ITEMS || px < FWD_LINE_PIXELS) return false;
+    if (g.shear_waves == 0 || 64 * g.shear_waves > FWD_LINE_ITEMS) return false;
     if (alone) return 24 * groups <= px && S * px <= (1ll << 25);
     return !P.fuse_primal && S <= 64 && groups <= 960 && 17 * groups <= px;
 }
@@ -974,7 +974,7 @@ static int fwd_line_k(const ProbDev& P, const Geometry& g, int nslices, int mode
 int launch_fwd(const ProbDev& P, const Geometry& g, int nslices, int mode, hipStream_t st)
 {
     if (nslices <= 0) return GR_OK;
-    if ((mode & FWD_SCRATCH) &&
+    if ((mode & FWD_SCRATCH) && P.shear &&
         ((mode & FWD_LINES) || fwd_by_lines(P, g, mode & FWD_ALONE))) {
         // fewer slices per work-group where angles x groups would not give
         // every CU one: 317 x 317 x 3, 71 angles, 10 iterations 1000 / 932 /

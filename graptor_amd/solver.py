@@ -136,6 +136,7 @@ class TgvProblem:
                                   device=self.device)
             self.k = StepConstants.make(self.dim, float(L), self.alpha, self.mu, discrepancy)
             self._alloc(u0)
+            geometry.prepare(self.C * self.Nz)
 
     # ------------------------------------------------------------------
     def _alloc(self, u0):
