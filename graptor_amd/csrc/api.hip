@@ -471,6 +471,7 @@ struct gr_plan {
     // mi: items per thread, or 0: by lines, in work-groups of `waves` waves
     struct FwdLaunch {
         int K, mi; size_t lds; std::vector<FwdItem> items; FwdItem* dev; int waves = 0;
+        bool wide = false;
     };
     struct AdjLaunch { int K, dim, tgv, fuse; size_t lds; std::vector<AdjItem> items; AdjItem* dev; };
     struct PrimalLaunch { int dim, tgv; std::vector<DualItem> items; DualItem* dev; };
@@ -543,6 +544,7 @@ int plan_build(gr_plan* pl, const gr_geometry* const* geoms)
                 tsel[i] = tt;
             }
         }
+        if (g.wide_bins) tsel[i] = FWD_WIDE_TABLE;
     }
     // waves per work-group of the launches by lines
     int line_waves = FWD_LINE_WAVES;
@@ -553,7 +555,7 @@ int plan_build(gr_plan* pl, const gr_geometry* const* geoms)
             set_shear(pl->probs[i], geoms[i]->g);
             line_waves = std::max(line_waves, geoms[i]->g.shear_waves);
         }
-    std::map<std::tuple<int, int>, size_t> fwd_idx;
+    std::map<std::tuple<int, int, int>, size_t> fwd_idx;
     std::map<std::tuple<int, int, int, int>, size_t> adj_idx;
     std::map<std::tuple<int, int>, size_t> primal_idx;
     std::map<std::tuple<int, int, int, int>, size_t> dual_idx;
@@ -565,7 +567,7 @@ int plan_build(gr_plan* pl, const gr_geometry* const* geoms)
         if (fwd_by_lines(P, g)) {
             // slice groups x runs of angles that fill line_waves waves of items
             const int J = g.shear_waves;
-            auto fk = std::make_tuple(K, 0);
+            auto fk = std::make_tuple(K, 0, 0);
             if (!fwd_idx.count(fk)) {
                 fwd_idx[fk] = pl->fwd.size();
                 pl->fwd.push_back({K, 0, 0, {}, nullptr});
@@ -583,10 +585,11 @@ int plan_build(gr_plan* pl, const gr_geometry* const* geoms)
         } else {
             // slice groups x chunks (group-major)
             const int t = tsel[i], mi = 8 >> t;
-            auto fk = std::make_tuple(K, mi);
+            auto fk = std::make_tuple(K, mi, g.wide_bins);
             if (!fwd_idx.count(fk)) {
                 fwd_idx[fk] = pl->fwd.size();
                 pl->fwd.push_back({K, mi, 0, {}, nullptr});
+                pl->fwd.back().wide = g.wide_bins != 0;
             }
             auto& fl = pl->fwd[fwd_idx[fk]];
             fl.lds = std::max(fl.lds, fwd_lds_bytes(P, K));
@@ -765,8 +768,8 @@ int plan_phase(gr_plan* pl, int phase, int fwd_mode, hipStream_t st)
                 rc = launch_fwd_line_batch(pl->probs_dev, l.dev, (int)l.items.size(), l.K,
                                            l.waves, fwd_mode, s);
             else
-                rc = launch_fwd_batch(pl->probs_dev, l.dev, (int)l.items.size(), l.K, l.mi, l.lds,
-                                      fwd_mode, s);
+                rc = launch_fwd_batch(pl->probs_dev, l.dev, (int)l.items.size(), l.K, l.mi,
+                                      l.wide, l.lds, fwd_mode, s);
         } else if (ph == 2) {
             const auto& l = pl->adj[i];
             rc = launch_adj_batch(pl->probs_dev, l.dev, (int)l.items.size(), l.K, l.dim,
@@ -887,7 +890,7 @@ int gr_geometry_create(const float* ofs, int na, int nx, int ny, int nd, gr_geom
     g.adj_tile_y = std::max(nx, ny) <= 256 ? 16 : 32;
     g.fuse_primal = 0;
     g.ofs_dev = nullptr; g.fwd_dev = nullptr; g.chunks_dev = nullptr;
-    g.narrow_bins = 0;
+    g.narrow_bins = g.wide_bins = 0;
     std::vector<FwdAngle> fa(na);
     for (int j = 0; j < na; ++j) {
         const double c = ofs[4 * j], s = ofs[4 * j + 1], o = ofs[4 * j + 2];
@@ -903,6 +906,7 @@ int gr_geometry_create(const float* ofs, int na, int nx, int ny, int nd, gr_geom
         a.mstep = (float)(a.cls == 0 ? c : s);
         a.mcand = (float)mc;
         a.off = (float)o;
+        if (std::fabs((double)a.mcand) < 2.0 / 3.0) g.wide_bins = 1;
         a.invc = (float)(1.0 / (double)a.mcand);
         a.hc = (float)(1.0 / std::fabs((double)a.mcand));
         a.id = j;

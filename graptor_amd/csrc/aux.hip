@@ -38,8 +38,10 @@ __device__ __forceinline__ double block_sum64(double v, double* red)
 // Forward projection of img / n, n the sum of the partial sums (root: its
 // square root), for 64 bins of an angle; the same hat-weight gather as the
 // FP32 kernel, with four candidates so that any rounding of the float
-// constants is tolerated.  Candidates are contiguous: rows of the image, or of
-// its transpose where the lines are columns.
+// constants is tolerated (WIDE: bins of more pixels, as many as their hats
+// reach over).  Candidates are contiguous: rows of the image, or of its
+// transpose where the lines are columns.
+template <bool WIDE>
 __global__ __launch_bounds__(T64) void fwd64_kernel(const double* __restrict__ img,
                                                     const double* __restrict__ imgt,
                                                     double* __restrict__ sino,
@@ -61,6 +63,15 @@ __global__ __launch_bounds__(T64) void fwd64_kernel(const double* __restrict__ i
 #pragma unroll 2
     for (int l = wave; l < len_step; l += W64) {
         const double r = (double)l * ms + ro;
+        if constexpr (WIDE) {
+            const double* __restrict__ line = src + (size_t)l * len_cand;
+            const double hi = (double)len_cand;
+            const int b = (int)fmin(fmax(ceil(-r * inv - half) - 1.0, 0.0), hi);
+            const int e = (int)fmin(fmax(floor(-r * inv + half) + 2.0, 0.0), hi);
+            for (int c = b; c < e; ++c)
+                acc += fmax(1.0 - fabs((double)c * mc + r), 0.0) * line[c];
+            continue;
+        }
         const double first = fmin(fmax(ceil(-r * inv - half) - 1.0, -4.0), (double)len_cand);
         const int b = (int)first;
         const double* __restrict__ line = src + (size_t)l * len_cand;
@@ -211,7 +222,7 @@ int launch_normest(const Geometry& g, const double* x0_host, int iters, int mode
     if (rc == GR_OK) image(nullptr, nullptr);
     double result = 0.0, prev = 0.0, h[2] = {0.0, 0.0};  // norm, dot
     for (int it = 0; it < iters && rc == GR_OK; ++it) {
-        hipLaunchKernelGGL(fwd64_kernel, dim3(fb), dim3(T64), 0, st, x, xt, s, g.fwd_dev, g.nx,
+        hipLaunchKernelGGL(g.wide_bins ? fwd64_kernel<true> : fwd64_kernel<false>, dim3(fb), dim3(T64), 0, st, x, xt, s, g.fwd_dev, g.nx,
                            g.ny, g.nd, parts, np, power ? 1 : 0, red);
         image(s, power ? dots : nullptr);
         chk(hipGetLastError(), "normest launch");

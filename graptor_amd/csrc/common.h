@@ -110,6 +110,10 @@ struct AdjItem { int prob, x0, y0, s0; };
 // z + nz * channel (primal step).
 struct DualItem { int prob, x0, y0, z; };
 
+// Chunk table (FWD_THREADS x 8 >> t items) of geometries with wide bins, the only
+// one whose gather is built for them.
+constexpr int FWD_WIDE_TABLE = 2;
+
 constexpr int SHEAR_BLOCK = 8;       // lines per table read
 constexpr double FWD_SHEAR_MIN = 0.7;
 constexpr int FWD_LINE_ITEMS = 1024;  // items of an angle: 16 waves
@@ -143,6 +147,7 @@ struct Geometry {
     int fwd_band;            // lines per LDS band (0: automatic)
     int adj_tile_y;          // rows per backprojection tile
     int narrow_bins;         // detector width below one pixel
+    int wide_bins;           // some |mcand| below 2/3: hats over more than 3 candidates
     int fuse_primal;         // 1: primal step in the backprojection epilogue
 };
 
@@ -300,7 +305,7 @@ int launch_primal_part(const ProbDev& P, int part, hipStream_t st);
 
 // ---- launchers (batches: descriptor table + item table) -------------------
 int launch_fwd_batch(const ProbDev* probs_dev, const FwdItem* items, int nitems, int K,
-                     int mi, size_t lds, int mode, hipStream_t st);
+                     int mi, bool wide, size_t lds, int mode, hipStream_t st);
 // The sheared forward projection of batch problems: items {prob, J, first
 // angle, angles, 0, 0, s0} of K slices, J = waves of items of one angle and
 // angles * J <= waves; after launch_transpose_batch (items: 32 x 32 tiles x0,

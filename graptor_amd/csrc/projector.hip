@@ -294,9 +294,11 @@ __global__ __launch_bounds__(256) void transpose_batch_kernel(const ProbDev* __r
 // The K slices stream through LDS in bands of `band` lines of that axis; per
 // line every item reads the <= 3 candidates on the other axis whose hat
 // weight can be positive.  After the last band each item holds its complete
-// ray sum and applies the sinogram epilogue.
+// ray sum and applies the sinogram epilogue.  WIDE: detector bins of more than
+// 1.06 pixels, whose hats reach over more candidates (2 / |mcand|): a loop over
+// those that lie in the image.
 // --------------------------------------------------------------------------
-template <int K, int MI>
+template <int K, int MI, bool WIDE>
 __device__ __forceinline__ void fwd_body(const ProbDev& P, const FwdItem& I, int mode,
                                          float* sh)
 {
@@ -317,6 +319,7 @@ __device__ __forceinline__ void fwd_body(const ProbDev& P, const FwdItem& I, int
     // ceil(-r / mcand - hc) = ceil(xs * ta + tb).
     float acc[MI][K];
     float ms[MI], mc[MI], ro[MI], ta[MI], tb[MI];
+    float reach[WIDE ? MI : 1];  // candidates of a hat
 #pragma unroll
     for (int it = 0; it < MI; ++it) {
         const int item = tid + it * FWD_THREADS;
@@ -328,6 +331,7 @@ __device__ __forceinline__ void fwd_body(const ProbDev& P, const FwdItem& I, int
         ro[it] = A.off - fi;
         ta[it] = -A.mstep * A.invc;
         tb[it] = fmaf(-ro[it], A.invc, -A.hc);
+        if constexpr (WIDE) reach[it] = 2.f * A.hc;
 #pragma unroll
         for (int k = 0; k < K; ++k) acc[it][k] = 0.f;
     }
@@ -394,6 +398,22 @@ __device__ __forceinline__ void fwd_body(const ProbDev& P, const FwdItem& I, int
             float xs = (float)l0;  // exact integer-valued step coordinate
             for (int st = 0; st < band; ++st, xs += 1.f) {
                 const float r = fmaf(xs, ms[it], ro[it]);
+                if constexpr (WIDE) {
+                    // one more on either side, for the rounding of the bounds
+                    const float at = fmaf(xs, ta[it], tb[it]);
+                    const int first = (int)__builtin_amdgcn_fmed3f(ceilf(at) - 1.f, 0.f, cand_hi);
+                    const int end = (int)__builtin_amdgcn_fmed3f(floorf(at + reach[it]) + 2.f,
+                                                                 0.f, cand_hi);
+                    const float* line = sh + K * (st * pitch + FWD_PADL);
+                    for (int c = first; c < end; ++c) {
+                        const float d = fmaf((float)c, mc[it], r);
+                        const float w = __builtin_amdgcn_fmed3f(1.f - fabsf(d), 0.f, 1.f);
+                        const Pack<K> v = lds_load<K>(line, c);
+#pragma unroll
+                        for (int k = 0; k < K; ++k) acc[it][k] = fmaf(w, v.v[k], acc[it][k]);
+                    }
+                    continue;
+                }
                 float bf = ceilf(fmaf(xs, ta[it], tb[it]));
                 // clamp into [-3, len_cand] (bf is never NaN: finite operands)
                 bf = __builtin_amdgcn_fmed3f(bf, -3.f, cand_hi);
@@ -449,7 +469,7 @@ __device__ __forceinline__ void fwd_body(const ProbDev& P, const FwdItem& I, int
     }
 }
 
-template <int K, int MI>
+template <int K, int MI, bool WIDE>
 __global__ __launch_bounds__(FWD_THREADS) void fwd_single_kernel(ProbDev P,
                                                                  const FwdChunk* __restrict__ chunks,
                                                                  int nchunks, int mode)
@@ -458,10 +478,10 @@ __global__ __launch_bounds__(FWD_THREADS) void fwd_single_kernel(ProbDev P,
     const int work = xcd_work_id(blockIdx.x, gridDim.x);
     const FwdChunk ch = chunks[work % nchunks];
     const FwdItem I{0, ch.cls, ch.a0, ch.na, ch.b0, ch.nb, (work / nchunks) * K, 0};
-    fwd_body<K, MI>(P, I, mode, sh);
+    fwd_body<K, MI, WIDE>(P, I, mode, sh);
 }
 
-template <int K, int MI>
+template <int K, int MI, bool WIDE>
 __global__ __launch_bounds__(FWD_THREADS) void fwd_batch_kernel(const ProbDev* __restrict__ probs,
                                                                 const FwdItem* __restrict__ items,
                                                                 int mode)
@@ -471,7 +491,7 @@ __global__ __launch_bounds__(FWD_THREADS) void fwd_batch_kernel(const ProbDev* _
     // round-robin over the XCDs, which balances the load
     const FwdItem I = items[blockIdx.x];
     const ProbDev P = load_prob(probs, I.prob);
-    fwd_body<K, MI>(P, I, mode, sh);
+    fwd_body<K, MI, WIDE>(P, I, mode, sh);
 }
 
 // --------------------------------------------------------------------------
@@ -859,11 +879,11 @@ int slice_group(int nslices) { return nslices >= 3 ? 4 : (nslices == 2 ? 2 : 1);
 // --------------------------------------------------------------------------
 // single-problem launchers
 // --------------------------------------------------------------------------
-template <int K, int MI>
+template <int K, int MI, bool WIDE = false>
 static void fwd_single_launch(const ProbDev& P, const FwdChunk* chunks, int nchunks, int groups,
                               size_t lds, int mode, hipStream_t st)
 {
-    hipLaunchKernelGGL((fwd_single_kernel<K, MI>), dim3((unsigned)(groups * nchunks)),
+    hipLaunchKernelGGL((fwd_single_kernel<K, MI, WIDE>), dim3((unsigned)(groups * nchunks)),
                        dim3(FWD_THREADS), lds, st, P, chunks, nchunks, mode);
 }
 
@@ -886,6 +906,7 @@ static int fwd_single_k(const ProbDev& Pin, const Geometry& g, int nslices, int 
         return v == 8 ? 0 : v == 4 ? 1 : v == 2 ? 2 : v == 1 ? 3 : -1;
     }();
     if (forced >= 0) t = forced;
+    if (g.wide_bins) t = FWD_WIDE_TABLE;
     const int nchunks = g.tab_off[t + 1] - g.tab_off[t];
     const FwdChunk* chunks = g.chunks_dev + g.tab_off[t];
     P.fwd_pitch = fwd_pitch_of(P.nx, P.ny);
@@ -911,7 +932,9 @@ static int fwd_single_k(const ProbDev& Pin, const Geometry& g, int nslices, int 
         set_error("radon: invalid grid (%lld blocks)", blocks);
         return GR_ERR_INVALID;
     }
-    switch (t) {
+    if (g.wide_bins)
+        fwd_single_launch<K, (8 >> FWD_WIDE_TABLE), true>(P, chunks, nchunks, groups, lds, mode, st);
+    else switch (t) {
     case 0: fwd_single_launch<K, 8>(P, chunks, nchunks, groups, lds, mode, st); break;
     case 1: fwd_single_launch<K, 4>(P, chunks, nchunks, groups, lds, mode, st); break;
     case 2: fwd_single_launch<K, 2>(P, chunks, nchunks, groups, lds, mode, st); break;
@@ -1259,14 +1282,17 @@ int launch_primal_batch(const ProbDev* probs, const DualItem* items, int nitems,
 // batch launchers
 // --------------------------------------------------------------------------
 int launch_fwd_batch(const ProbDev* probs, const FwdItem* items, int nitems, int K, int mi,
-                     size_t lds, int mode, hipStream_t st)
+                     bool wide, size_t lds, int mode, hipStream_t st)
 {
     if (nitems <= 0) return GR_OK;
     dim3 grd((unsigned)nitems), blk(FWD_THREADS);
 #define GR_FB(KK, MM) \
-    hipLaunchKernelGGL((fwd_batch_kernel<KK, MM>), grd, blk, lds, st, probs, items, mode)
+    hipLaunchKernelGGL((fwd_batch_kernel<KK, MM, false>), grd, blk, lds, st, probs, items, mode)
 #define GR_FB_K(KK)                                  \
-    switch (mi) {                                    \
+    if (wide)                                        \
+        hipLaunchKernelGGL((fwd_batch_kernel<KK, (8 >> FWD_WIDE_TABLE), true>), grd, blk, lds, st, \
+                           probs, items, mode);      \
+    else switch (mi) {                               \
     case 8: GR_FB(KK, 8); break;                     \
     case 4: GR_FB(KK, 4); break;                     \
     case 2: GR_FB(KK, 2); break;                     \
