@@ -290,8 +290,8 @@ ProbDev make_prob(const gr_geometry* gg, const gr_tgv_params* p, const gr_tgv_st
     P.fwd_pitch = fwd_pitch_of(g.nx, g.ny);
     P.fwd_band = g.fwd_band > 0 ? g.fwd_band : fwd_band_auto(P.fwd_pitch, K);
     P.adj_tile_y = g.adj_tile_y;
-    P.narrow_bins = g.narrow_bins;
-    P.adj_segw = adj_segw_of(P.adj_tile_y);
+    P.bin_span = g.bin_span;
+    P.adj_segw = adj_segw_of(P.adj_tile_y, P.bin_span);
     P.adj_achunk = adj_achunk_of(g.na, P.adj_segw, K);
     P.fuse_primal = g.fuse_primal;
     P.ofs = reinterpret_cast<const float4*>(g.ofs_dev);
@@ -607,6 +607,10 @@ int plan_build(gr_plan* pl, const gr_geometry* const* geoms)
         }
         auto& al = pl->adj[adj_idx[ak]];
         al.lds = std::max(al.lds, adj_lds_bytes(P, K));
+        if (al.lds > LDS_LIMIT) {
+            set_error("plan: bins of 1/%.0f pixel are too narrow for a batch", P.bin_span);
+            return GR_ERR_INVALID;
+        }
         for (int s0 = 0; s0 < S; s0 += K)
             for (int y0 = 0; y0 < P.ny; y0 += P.adj_tile_y)
                 for (int x0 = 0; x0 < P.nx; x0 += ADJ_TX) al.items.push_back(AdjItem{i, x0, y0, s0});
@@ -647,7 +651,7 @@ int plan_build(gr_plan* pl, const gr_geometry* const* geoms)
                          [&](const FwdItem& a, const FwdItem& b) { return work(a) > work(b); });
     }
     for (auto& l : pl->fwd)
-        if (l.lds > 160 * 1024) {
+        if (l.lds > LDS_LIMIT) {
             set_error("plan: forward LDS stage of %zu bytes too large", l.lds);
             return GR_ERR_INVALID;
         }
@@ -831,7 +835,7 @@ ProbDev standalone(const gr_geometry* gg, int nslices)
     P.fwd = g.fwd_dev;
     P.fwd_band = g.fwd_band;
     P.adj_tile_y = g.adj_tile_y;
-    P.narrow_bins = g.narrow_bins;
+    P.bin_span = g.bin_span;
     return P;
 }
 
@@ -890,11 +894,14 @@ int gr_geometry_create(const float* ofs, int na, int nx, int ny, int nd, gr_geom
     g.adj_tile_y = std::max(nx, ny) <= 256 ? 16 : 32;
     g.fuse_primal = 0;
     g.ofs_dev = nullptr; g.fwd_dev = nullptr; g.chunks_dev = nullptr;
-    g.narrow_bins = g.wide_bins = 0;
+    g.wide_bins = 0;
+    g.bin_span = 1.f;
     std::vector<FwdAngle> fa(na);
     for (int j = 0; j < na; ++j) {
         const double c = ofs[4 * j], s = ofs[4 * j + 1], o = ofs[4 * j + 2];
-        if (std::hypot(c, s) > 1.0 + 1e-5) g.narrow_bins = 1;
+        // unit bins are off one by the rounding of the table
+        if (std::hypot(c, s) > 1.0 + 1e-5)
+            g.bin_span = std::max(g.bin_span, (float)std::hypot(c, s));
         FwdAngle a{};
         a.cls = std::fabs(s) >= std::fabs(c) ? 0 : 1;
         const double mc = a.cls == 0 ? s : c;
@@ -1371,7 +1378,7 @@ int gr_plan_retune(gr_plan* pl, const gr_geometry* const* geoms)
         const int K = slice_group(P.nz * P.nch);
         P.fwd_band = g.fwd_band > 0 ? g.fwd_band : fwd_band_auto(P.fwd_pitch, K);
         P.adj_tile_y = g.adj_tile_y;
-        P.adj_segw = adj_segw_of(P.adj_tile_y);
+        P.adj_segw = adj_segw_of(P.adj_tile_y, P.bin_span);
         P.adj_achunk = adj_achunk_of(g.na, P.adj_segw, K);
         P.fuse_primal = g.fuse_primal;
     }

@@ -86,7 +86,7 @@ struct ProbDev {
     const int* line0;
     const FwdBin* bins;
     int shear_stride;
-    int narrow_bins;       // a step of one pixel may cross more than one bin
+    float bin_span;        // most bins that a step of one pixel crosses, at least 1
     // state; for standalone projector calls: ubar = image in, ku = sinogram
     // out (forward), lam = sinogram in, ktl = image out (backprojection)
     float *u, *ubar, *p, *pbar, *v, *w, *lam, *ktl, *ku;
@@ -146,7 +146,7 @@ struct Geometry {
     int shear_stride;
     int fwd_band;            // lines per LDS band (0: automatic)
     int adj_tile_y;          // rows per backprojection tile
-    int narrow_bins;         // detector width below one pixel
+    float bin_span;          // most bins that a step of one pixel crosses, at least 1
     int wide_bins;           // some |mcand| below 2/3: hats over more than 3 candidates
     int fuse_primal;         // 1: primal step in the backprojection epilogue
 };
@@ -271,10 +271,11 @@ inline void set_shear(ProbDev& P, const Geometry& g)  // after line_tables
 int fwd_pitch_of(int nx, int ny);
 int fwd_table_choice(const Geometry& g, long long groups, double wg_per_cu = 3.0);
 int fwd_band_auto(int pitch, int K, int lds_kb = 36);
-int adj_segw_of(int tile_y);
+int adj_segw_of(int tile_y, float bin_span);
 int adj_achunk_of(int na, int segw, int K);
 size_t fwd_lds_bytes(const ProbDev& P, int K);
 size_t adj_lds_bytes(const ProbDev& P, int K);
+constexpr size_t LDS_LIMIT = 160 * 1024;  // of a work-group
 int slice_group(int nslices);  // K = 4 (3 or more slices), 2 or 1 slices sharing geometry
 
 // ---- launchers (single problem: descriptor by value) ---------------------

@@ -836,11 +836,12 @@ int fwd_band_auto(int pitch, int K, int lds_kb)
     return std::max(4, std::min(32, b & ~3));
 }
 
-int adj_segw_of(int tile_y)
+int adj_segw_of(int tile_y, float bin_span)
 {
     const double diag = std::sqrt((double)(ADJ_TX - 1) * (ADJ_TX - 1) +
                                   (double)(tile_y - 1) * (tile_y - 1));
-    int w = (int)std::ceil(diag) + 6;
+    // capped past what LDS can hold
+    int w = (int)std::ceil(std::min(diag * bin_span, 1e6)) + 6;
     return (w + 3) & ~3;
 }
 
@@ -923,7 +924,7 @@ static int fwd_single_k(const ProbDev& Pin, const Geometry& g, int nslices, int 
         P.fwd_band = fwd_band_auto(P.fwd_pitch, K, (int)(160 / per_cu) - 1);
     }
     const size_t lds = fwd_lds_bytes(P, K);
-    if (lds > 160 * 1024) {
+    if (lds > LDS_LIMIT) {
         set_error("radon: band %d does not fit LDS (%zu bytes)", P.fwd_band, lds);
         return GR_ERR_INVALID;
     }
@@ -1046,9 +1047,14 @@ static int adj_single_k(const ProbDev& Pin, int nslices, bool primal, hipStream_
                   4 * ADJ_MAXR);
         return GR_ERR_INVALID;
     }
-    P.adj_segw = adj_segw_of(P.adj_tile_y);
+    P.adj_segw = adj_segw_of(P.adj_tile_y, P.bin_span);
     P.adj_achunk = adj_achunk_of(P.na, P.adj_segw, K);
     const size_t lds = adj_lds_bytes(P, K);
+    if (lds > LDS_LIMIT) {
+        set_error("radon_ad: bins of 1/%.0f pixel are too narrow for the fused primal step",
+                  P.bin_span);
+        return GR_ERR_INVALID;
+    }
     const int tiles_x = (P.nx + ADJ_TX - 1) / ADJ_TX;
     const int tiles_y = (P.ny + P.adj_tile_y - 1) / P.adj_tile_y;
     const int ntiles = tiles_x * tiles_y;
@@ -1102,14 +1108,17 @@ static int adj_direct_k(const ProbDev& P, int nslices, bool u_half, hipStream_t 
 // 58 / 45 / 39 to 33; 512 x 512 x 1 12 to 33, x 4 31 / 25 / 24 to 35.
 // Whole iterations: 183 x 183 x 16 71 to 78, 512 x 512 x 4 94 to 109, but
 // 64 x 64 x 256 (256 work-groups) 89 to 86, 256 x 256 x 24 (384) 116 to 108.
-// Bins narrower than a pixel stay with the tiles at every size.
+// Bins so narrow that not one angle's shadow of a tile fits LDS are read
+// directly at every size.
 // Returns the slices per wave, 0: by tiles.
 static int adj_direct_slices(const ProbDev& P, int nslices, bool wide)
 {
-    if (P.narrow_bins || P.adj_tile_y < 4 || P.adj_tile_y % 4 != 0) return 0;
+    if (P.adj_tile_y < 4 || P.adj_tile_y % 4 != 0) return 0;
     const long long cols = (P.nx + ADJ_TX - 1) / ADJ_TX, rows = cols * P.ny;
     const long long tiles = cols * ((P.ny + P.adj_tile_y - 1) / P.adj_tile_y);
     const int K = wide ? 8 : slice_group(nslices);
+    const size_t shadow = (size_t)adj_segw_of(P.adj_tile_y, P.bin_span) * K * sizeof(float);
+    if (shadow + sizeof(float4) + sizeof(int) > LDS_LIMIT) return slice_group(nslices);
     if (tiles * ((nslices + K - 1) / K) >= 256) return 0;
     for (int d = 1; d <= 4; d *= 2)
         if (rows * ((nslices + d - 1) / d) <= 6144) return d;
