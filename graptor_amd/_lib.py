@@ -28,7 +28,7 @@ HALO_PHASE = {"dual": 0, "primal": 1}
 EXPORTS = (
     "gr_last_error", "gr_abi_version", "gr_radon_struct", "gr_geometry_create",
     "gr_geometry_destroy", "gr_geometry_set_tuning", "gr_geometry_get_tuning",
-    "gr_geometry_set_fusion", "gr_geometry_prepare", "gr_iterates_by_lines",
+    "gr_geometry_set_fusion", "gr_iterates_by_lines",
     "gr_radon", "gr_radon_scratch", "gr_radon_scratch_floats", "gr_radon_ad", "gr_normest", "gr_make_feasible", "gr_tgv_iterate",
     "gr_tgv_energy", "gr_tgv_profile", "gr_plan_create", "gr_plan_destroy",
     "gr_plan_iterate", "gr_plan_iterate_graph", "gr_plan_profile", "gr_plan_retune",
@@ -96,7 +96,6 @@ def load(path: str | None = None):
             "gr_geometry_set_tuning": ([V, I, I], I),
             "gr_geometry_get_tuning": ([V, PI, PI], I),
             "gr_geometry_set_fusion": ([V, I], I),
-            "gr_geometry_prepare": ([V, I], I),
             "gr_iterates_by_lines": ([V, I], I),
             "gr_radon": ([V, V, V, I, V], I),
             "gr_radon_scratch": ([V, V, V, I, V, I, V], I),

@@ -8,7 +8,6 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
-#include <memory>
 #include <new>
 #include <tuple>
 #include <vector>
@@ -97,133 +96,38 @@ ItemRange items_of(const FwdAngle& A, int nd)
     return r;
 }
 
-int shear_waves_of(const std::vector<FwdAngle>& fa, int nx, int ny, int nd)
-{
-    if (nd + 2 > FWD_LINE_ITEMS || (long long)nx * ny < FWD_LINE_PIXELS) return 0;
+// First item of each angle, items of the angles before it (and of all), and the
+// waves of the angle with the most: 0 where the sheared projection does not apply.
+struct ItemTable {
+    std::vector<int> first, line0;
     int waves = 0;
-    for (const FwdAngle& A : fa) {
-        const double m = std::fabs((double)A.mcand);
-        if (!(m >= FWD_SHEAR_MIN && m <= 1.0 && std::fabs((double)A.off) < 1e6)) return 0;
-        const ItemRange r = items_of(A, nd);
-        waves = std::max(waves, (int)((r.last - r.first + 64) / 64));
-    }
-    return waves;
-}
-
-// Its tables (FwdLine, FwdBin, Shear of common.h) in one block of memory, at
-// these offsets.
-struct ShearTables {
-    size_t shear, lines, line0, bins, bytes;
-    std::unique_ptr<char[]> mem;
-    template <typename T>
-    T* at(size_t offset) const { return reinterpret_cast<T*>(mem.get() + offset); }
 };
 
-ShearTables make_shear(const std::vector<FwdAngle>& fa, int nd, int nlines)
+ItemTable item_table(const std::vector<FwdAngle>& fa, int nx, int ny, int nd)
 {
-    const int na = (int)fa.size();
-    std::vector<ItemRange> range(na);
-    size_t items = 0;
-    for (int a = 0; a < na; ++a) {
-        range[a] = items_of(fa[a], nd);
-        items += (size_t)(range[a].last - range[a].first + 1);
-    }
-    ShearTables T;
-    T.shear = 0;
-    T.lines = T.shear + sizeof(Shear) * na * nlines;
-    T.bins = T.lines + sizeof(FwdLine) * items;
-    T.line0 = T.bins + sizeof(FwdBin) * na * nd;
-    T.bytes = T.line0 + sizeof(int) * (na + 1);
-    T.mem.reset(new char[T.bytes]);
-    FwdLine* line = T.at<FwdLine>(T.lines);
-    int* line0 = T.at<int>(T.line0);
-    std::vector<int> at(nd);  // bits taken of a bin's code
-    line0[0] = 0;
-    for (int a = 0; a < na; ++a) {
-        const double ms = fa[a].mstep, mc = fa[a].mcand, off = fa[a].off, inv = 1.0 / mc;
-        const ItemRange r = range[a];
-        FwdBin* bins = T.at<FwdBin>(T.bins) + (size_t)a * nd;
-        std::fill(bins, bins + nd, FwdBin{0, 0});
-        std::fill(at.begin(), at.end(), 0);
-        for (long long j = r.first; j <= r.last; ++j) {
-            const double t = (double)j * mc + off;
-            const int m = (int)nearest(t), i = (int)(j - r.first);
-            *line++ = FwdLine{(int)j, (float)(t - (double)m)};
-            for (int b = std::max(0, m - 1); b <= std::min(nd - 1, m + 1); ++b) {
-                if (at[b] == 0) bins[b].first = i;
-                bins[b].code |= (b - m + 2) << at[b];
-                at[b] += 3;
-            }
-        }
-        line0[a + 1] = line0[a] + (int)(r.last - r.first + 1);
-        Shear* shear = T.at<Shear>(T.shear) + (size_t)a * nlines;
-        for (int l = 0; l < nlines; ++l) {
-            const long long s = nearest(-l * ms * inv);
-            shear[l] = Shear{(float)(l * ms + (double)s * mc), (int)s};
-        }
+    ItemTable T, none;
+    if (nd + 2 > FWD_LINE_ITEMS || (long long)nx * ny < FWD_LINE_PIXELS) return none;
+    T.line0.push_back(0);
+    for (const FwdAngle& A : fa) {
+        const double m = std::fabs((double)A.mcand);
+        if (!(m >= FWD_SHEAR_MIN && m <= 1.0 && std::fabs((double)A.off) < 1e6)) return none;
+        const ItemRange r = items_of(A, nd);
+        const int n = (int)(r.last - r.first + 1);
+        T.first.push_back((int)r.first);
+        T.line0.push_back(T.line0.back() + n);
+        T.waves = std::max(T.waves, (n + 63) / 64);
     }
     return T;
 }
 
 template <typename T>
-int upload(const T* v, size_t n, T** out)
+int upload(const std::vector<T>& v, T** out)
 {
     *out = nullptr;
-    if (n == 0) return GR_OK;
-    GR_HIP(hipMalloc(out, sizeof(T) * n));
-    GR_HIP(hipMemcpy(*out, v, sizeof(T) * n, hipMemcpyHostToDevice));
+    if (v.empty()) return GR_OK;
+    GR_HIP(hipMalloc(out, sizeof(T) * v.size()));
+    GR_HIP(hipMemcpy(*out, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
     return GR_OK;
-}
-
-template <typename T>
-int upload(const std::vector<T>& v, T** out) { return upload(v.data(), v.size(), out); }
-
-// The tables of the projection by lines: built and copied by the first call that
-// projects so, or ahead of it by gr_geometry_prepare.  Large stacks,
-// backprojections and operator norms never need them, and they are most of a
-// geometry: 256 x 256, 60 angles 0.14 ms and 0.4 MB, 512 x 512, 120 angles 0.6 ms
-// and 1.6 MB.  Not while `st` is captured (memory cannot be allocated then): such
-// a call gathers.  GR_OK without tables: it gathers too.
-int line_tables(const Geometry& g, hipStream_t st, bool on_stream = true)
-{
-    if (g.shear_waves == 0 || g.shear_ready.load(std::memory_order_acquire)) return GR_OK;
-    if (on_stream) {
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone)
-            return GR_OK;
-    }
-    try {
-        std::lock_guard<std::mutex> hold(g.shear_mutex);
-        if (g.shear_ready.load(std::memory_order_relaxed)) return GR_OK;
-        const ShearTables T = make_shear(g.fwd_host, g.nd, g.shear_stride);
-        int dev = 0;
-        GR_HIP(hipGetDevice(&dev));
-        if (dev != g.device) GR_HIP(hipSetDevice(g.device));
-        char* at = nullptr;
-        const int rc = upload(T.mem.get(), T.bytes, &at);
-        if (dev != g.device) (void)hipSetDevice(dev);
-        if (rc) {
-            if (at) (void)hipFree(at);
-            return rc;
-        }
-        g.shear_dev = reinterpret_cast<Shear*>(at + T.shear);
-        g.lines_dev = reinterpret_cast<const FwdLine*>(at + T.lines);
-        g.line0_dev = reinterpret_cast<const int*>(at + T.line0);
-        g.bins_dev = reinterpret_cast<const FwdBin*>(at + T.bins);
-        g.shear_ready.store(true, std::memory_order_release);
-    } catch (const std::exception&) {
-        set_error("line_tables: host allocation failed");
-        return GR_ERR_OOM;
-    }
-    return GR_OK;
-}
-
-// Tables into P where they are there (all: or can be had) for a projection by
-// lines; one that cannot have them gathers.
-void want_lines(ProbDev& P, const Geometry& g, hipStream_t st)
-{
-    if (line_tables(g, st) != GR_OK) (void)hipGetLastError();
-    if (g.shear_ready.load(std::memory_order_acquire)) set_shear(P, g);
 }
 
 hipStream_t stream_of(void* s) { return reinterpret_cast<hipStream_t>(s); }
@@ -296,6 +200,7 @@ ProbDev make_prob(const gr_geometry* gg, const gr_tgv_params* p, const gr_tgv_st
     P.fuse_primal = g.fuse_primal;
     P.ofs = reinterpret_cast<const float4*>(g.ofs_dev);
     P.fwd = g.fwd_dev;
+    set_shear(P, g);
     P.u = s->u; P.ubar = s->ubar; P.p = s->p; P.pbar = s->pbar; P.v = s->v; P.w = s->w;
     P.lam = s->lam; P.ktl = s->ktl; P.ku = s->ku; P.f = s->f; P.mfac = s->mfac;
     P.halo_ubar_hi = s->halo_ubar_hi; P.halo_pbar_lo = s->halo_pbar_lo;
@@ -549,12 +454,8 @@ int plan_build(gr_plan* pl, const gr_geometry* const* geoms)
     // waves per work-group of the launches by lines
     int line_waves = FWD_LINE_WAVES;
     for (int i = 0; i < n; ++i)
-        if (fwd_by_lines(pl->probs[i], geoms[i]->g)) {
-            const int lrc = line_tables(geoms[i]->g, nullptr, false);
-            if (lrc) return lrc;
-            set_shear(pl->probs[i], geoms[i]->g);
+        if (fwd_by_lines(pl->probs[i], geoms[i]->g))
             line_waves = std::max(line_waves, geoms[i]->g.shear_waves);
-        }
     std::map<std::tuple<int, int, int>, size_t> fwd_idx;
     std::map<std::tuple<int, int, int, int>, size_t> adj_idx;
     std::map<std::tuple<int, int>, size_t> primal_idx;
@@ -928,30 +829,53 @@ int gr_geometry_create(const float* ofs, int na, int nx, int ny, int nd, gr_geom
         g.chunks_host.insert(g.chunks_host.end(), c.begin(), c.end());
     }
     g.tab_off[4] = (int)g.chunks_host.size();
-    g.shear_waves = shear_waves_of(fa, nx, ny, nd);
+    const ItemTable items = item_table(fa, nx, ny, nd);
+    g.shear_waves = items.waves;
     g.shear_stride = std::max(nx, ny) + SHEAR_BLOCK;
-    // one allocation, owned by ofs_dev, and one copy for all tables
+    // one allocation, owned by ofs_dev: these tables, which one copy brings, and
+    // behind them the sheared projection's, filled on the device
     std::vector<char> all;
+    size_t bytes = 0;
+    auto room = [&](size_t n) {
+        const size_t at = bytes;
+        bytes = (at + n + 63) / 64 * 64;
+        return at;
+    };
     auto put = [&](const void* p, size_t n) {
-        const size_t at = all.size();
-        all.resize((at + n + 63) / 64 * 64);
-        std::memcpy(all.data() + at, p, n);
+        const size_t at = room(n);
+        all.resize(bytes);
+        if (n) std::memcpy(all.data() + at, p, n);
         return at;
     };
     put(ofs, sizeof(float) * 4 * na);
     const size_t fwd = put(fa.data(), sizeof(FwdAngle) * na);
     const size_t chunks = put(g.chunks_host.data(), sizeof(FwdChunk) * g.chunks_host.size());
+    const size_t line0 = put(items.line0.data(), sizeof(int) * items.line0.size());
+    const size_t first = put(items.first.data(), sizeof(int) * items.first.size());
+    size_t shear = 0, lines = 0, bins = 0;
+    if (items.waves) {
+        shear = room(sizeof(Shear) * na * g.shear_stride);
+        lines = room(sizeof(FwdLine) * items.line0[na]);
+        bins = room(sizeof(FwdBin) * na * nd);
+    }
     char* dev = nullptr;
-    int rc = upload(all, &dev);
+    hipError_t e = hipMalloc(&dev, bytes);
     g.ofs_dev = reinterpret_cast<float*>(dev);
-    if (!rc && hipGetDevice(&g.device) != hipSuccess) rc = hip_status(hipGetLastError(), "device");
+    if (e == hipSuccess) e = hipMemcpy(dev, all.data(), all.size(), hipMemcpyHostToDevice);
+    int rc = e == hipSuccess ? GR_OK : hip_status(e, "geometry_create");
+    g.fwd_dev = reinterpret_cast<FwdAngle*>(dev + fwd);
+    g.chunks_dev = reinterpret_cast<FwdChunk*>(dev + chunks);
+    if (items.waves) {
+        g.shear_dev = reinterpret_cast<Shear*>(dev + shear);
+        g.lines_dev = reinterpret_cast<FwdLine*>(dev + lines);
+        g.line0_dev = reinterpret_cast<int*>(dev + line0);
+        g.bins_dev = reinterpret_cast<FwdBin*>(dev + bins);
+        if (!rc) rc = launch_line_tables(g, reinterpret_cast<const int*>(dev + first));
+    }
     if (rc) {
         gr_geometry_destroy(gg);
         return rc;
     }
-    g.fwd_dev = reinterpret_cast<FwdAngle*>(dev + fwd);
-    g.chunks_dev = reinterpret_cast<FwdChunk*>(dev + chunks);
-    if (g.shear_waves) g.fwd_host = std::move(fa);
     *out = gg;
     return GR_OK;
 }
@@ -961,7 +885,6 @@ int gr_geometry_destroy(gr_geometry* gg)
     if (!gg) return GR_OK;
     Geometry& g = gg->g;
     if (g.ofs_dev) (void)hipFree(g.ofs_dev);
-    if (g.shear_dev) (void)hipFree(g.shear_dev);
     delete gg;
     return GR_OK;
 }
@@ -990,17 +913,6 @@ int gr_geometry_set_fusion(gr_geometry* gg, int fuse_primal)
     }
     gg->g.fuse_primal = fuse_primal;
     return GR_OK;
-}
-
-int gr_geometry_prepare(const gr_geometry* gg, int nslices)
-{
-    if (!gg || nslices <= 0) {
-        set_error("geometry_prepare: invalid arguments");
-        return GR_ERR_INVALID;
-    }
-    const ProbDev P = standalone(gg, nslices);
-    if (!fwd_by_lines(P, gg->g) && !fwd_by_lines(P, gg->g, true)) return GR_OK;
-    return line_tables(gg->g, nullptr, false);
 }
 
 int gr_iterates_by_lines(const gr_geometry* gg, int nslices)
@@ -1049,6 +961,7 @@ int gr_radon_scratch(const gr_geometry* gg, float* sino, const float* img, int n
         return GR_ERR_INVALID;
     }
     ProbDev P = standalone(gg, nslices);
+    set_shear(P, gg->g);
     P.ubar = const_cast<float*>(img);
     P.ku = sino;
     P.ktl = scratch;
@@ -1062,7 +975,6 @@ int gr_radon_scratch(const gr_geometry* gg, float* sino, const float* img, int n
         set_error("radon_scratch: the scratch overlaps the image or the sinogram");
         return GR_ERR_INVALID;
     }
-    if (lines) want_lines(P, gg->g, stream_of(stream));
     return launch_fwd(P, gg->g, nslices, mode, stream_of(stream));
 }
 
@@ -1113,8 +1025,7 @@ int gr_tgv_iterate(const gr_geometry* gg, const gr_tgv_params* p, const gr_tgv_s
         return GR_ERR_UNSUPPORTED;
     }
     if (n_iter == 0) return GR_OK;
-    ProbDev P = make_prob(gg, p, s);
-    if (fwd_by_lines(P, gg->g)) want_lines(P, gg->g, stream_of(stream));
+    const ProbDev P = make_prob(gg, p, s);
     return iterate_single(gg, P, n_iter, ku_on_last, stream_of(stream), nullptr, s);
 }
 
@@ -1155,8 +1066,7 @@ int gr_tgv_profile(const gr_geometry* gg, const gr_tgv_params* p, const gr_tgv_s
                   "run slabs through gr_tgv_dual_step / gr_tgv_primal_step");
         return GR_ERR_UNSUPPORTED;
     }
-    ProbDev P = make_prob(gg, p, s);
-    if (fwd_by_lines(P, gg->g)) want_lines(P, gg->g, stream_of(stream));
+    const ProbDev P = make_prob(gg, p, s);
     return iterate_single(gg, P, n_iter, 0, stream_of(stream), ms_out, s);
 }
 

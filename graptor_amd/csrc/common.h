@@ -4,8 +4,6 @@
 #include <stddef.h>
 #include <stdint.h>
 
-#include <atomic>
-#include <mutex>
 #include <vector>
 
 #include "../../include/graptor_amd.h"
@@ -129,20 +127,14 @@ struct Geometry {
     int tab_off[5];          // table t = chunks [tab_off[t], tab_off[t+1]),
                              // built for 8, 4, 2, 1 items per thread
     std::vector<FwdChunk> chunks_host;
-    // sheared projection: waves of items of the angle with the most, or 0 where
-    // it does not apply (every |mcand| in [FWD_SHEAR_MIN, 1], i.e. unit
-    // detector bins; see shear_waves_of)
+    // sheared projection: waves of items of the angle with the most, or 0 and no
+    // tables where it does not apply (every |mcand| in [FWD_SHEAR_MIN, 1], i.e.
+    // unit detector bins; see item_table)
     int shear_waves;
-    // its tables, one allocation owned by shear_dev: built by the first call
-    // that needs them (line_tables) and final once shear_ready is set
-    int device;
-    std::vector<FwdAngle> fwd_host;  // as fwd_dev
-    mutable std::mutex shear_mutex;
-    mutable std::atomic<bool> shear_ready{false};
-    mutable Shear* shear_dev = nullptr;      // na x shear_stride
-    mutable const FwdLine* lines_dev;
-    mutable const int* line0_dev;            // na + 1
-    mutable const FwdBin* bins_dev;          // na x nd
+    Shear* shear_dev = nullptr;  // na x shear_stride
+    FwdLine* lines_dev = nullptr;
+    int* line0_dev = nullptr;    // na + 1
+    FwdBin* bins_dev = nullptr;  // na x nd
     int shear_stride;
     int fwd_band;            // lines per LDS band (0: automatic)
     int adj_tile_y;          // rows per backprojection tile
@@ -261,7 +253,7 @@ __device__ __forceinline__ int stencil_block()
     return ((local / G) * 8 + xcd) * G + local % G;
 }
 
-inline void set_shear(ProbDev& P, const Geometry& g)  // after line_tables
+inline void set_shear(ProbDev& P, const Geometry& g)
 {
     P.shear = g.shear_dev; P.lines = g.lines_dev; P.line0 = g.line0_dev; P.bins = g.bins_dev;
     P.shear_stride = g.shear_stride;
@@ -317,10 +309,13 @@ int launch_fwd_batch(const ProbDev* probs_dev, const FwdItem* items, int nitems,
 constexpr int FWD_LINE_WAVES = 12;
 int launch_fwd_line_batch(const ProbDev* probs_dev, const FwdItem* items, int nitems, int K,
                           int waves, int mode, hipStream_t st);
+// Fills the tables of the sheared projection (line0 is there; first: each angle's
+// first item) and waits.
+int launch_line_tables(const Geometry& g, const int* first);
 int launch_transpose_batch(const ProbDev* probs_dev, const DualItem* items, int nitems,
                            hipStream_t st);
 // Whether an iteration of this problem (alone: a projection outside one)
-// projects forward by lines, given the tables (set_shear).
+// projects forward by lines.
 bool fwd_by_lines(const ProbDev& P, const Geometry& g, bool alone = false);
 int launch_adj_batch(const ProbDev* probs_dev, const AdjItem* items, int nitems, int K,
                      int dim, bool tgv, bool primal, size_t lds, hipStream_t st);

@@ -74,11 +74,6 @@ class RadonGeometry:
                    "get_tuning")
         return a.value, b.value
 
-    def prepare(self, nslices: int) -> None:
-        """Build now what projections of ``nslices`` slices need beyond the
-        geometry itself; the first of them does it otherwise."""
-        _lib.check(_lib.load().gr_geometry_prepare(self._h, int(nslices)), "geometry_prepare")
-
     def iterates_by_lines(self, nslices: int) -> bool:
         """Whether an iteration of ``nslices`` slices projects forward by lines
         (small stacks) instead of gathering each ray's pixels."""

@@ -136,7 +136,6 @@ class TgvProblem:
                                   device=self.device)
             self.k = StepConstants.make(self.dim, float(L), self.alpha, self.mu, discrepancy)
             self._alloc(u0)
-            geometry.prepare(self.C * self.Nz)
 
     # ------------------------------------------------------------------
     def _alloc(self, u0):

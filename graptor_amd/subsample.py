@@ -150,9 +150,6 @@ class SubsampledProblem:
                 f1[:, :, :, :min(nd, nd1)].masked_fill_(dead.view(1, 1, na1, -1), 0.0)
             self.f0, self.f1 = f0, f1
             self._alloc()
-            for g, C in ((self.g0, C0), (self.g1, C1)):
-                if C:
-                    g.prepare(C * nz)
             self.L = float(L) if L is not None else self.normest(seed=normest_seed)
         self.alpha = tuple(float(a) for a in alpha)
         self.mu = np.asarray(mu, np.float64).reshape(-1)

@@ -64,11 +64,6 @@ int gr_geometry_get_tuning(const gr_geometry *g, int *fwd_band, int *adj_tile_y)
  * stored); 0 (default): backprojection writes st->ktl and a separate
  * primal kernel reads it. */
 int gr_geometry_set_fusion(gr_geometry *g, int fuse_primal);
-/* Builds the tables that stacks of nslices slices need to be projected by lines
- * (0.14 ms for 256 x 256 and 60 angles, 0.6 ms for 512 x 512 and 120).  The first
- * such call does it by itself, except while its stream is captured: it gathers
- * then.  Plans bring theirs along. */
-int gr_geometry_prepare(const gr_geometry *g, int nslices);
 /* 1 if an iteration of nslices slices projects forward by lines (small stacks;
  * fwd_band has no part in it), 0 if it gathers each ray's pixels. */
 int gr_iterates_by_lines(const gr_geometry *g, int nslices);
