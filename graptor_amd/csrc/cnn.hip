@@ -244,7 +244,7 @@ __global__ __launch_bounds__(256) void conv_tile_kernel(
 // 142 to 104; 128 at 64 x 64 and 256 at 32 x 32: 161 to 78); 700 GFLOP, 580 us
 // at the rate of a large product.  Two output tiles per wave (TN = 2) spill at
 // 4 rows: the whole inference 1745 us with them at 64 x 64, 1886 at 32 x 32, 1651
-// with one.  What bounds it now: one or two work-groups per CU, whose staging is
+// with one, the only form launched (the same kernel without the parameter: 1661).  What bounds it now: one or two work-groups per CU, whose staging is
 // not all hidden, and at 256 x 256 memory (1.3 GB, 277 us at 4.6 TB/s, of 556).
 // ---------------------------------------------------------------------------
 template <int WAVES_M_, int TM_, int TN_, int KC_>

@@ -137,6 +137,11 @@ def radon(sino, img, r_struct, wait_for=None):
 
     ``wait_for`` is accepted for call-compatibility; ordering follows the
     current torch stream.  Returns None (the reference returns an event).
+
+    Small stacks are projected by lines, larger ones, and any while a graph is
+    captured, by gathering each ray's pixels.  The two sum in different orders,
+    so the last bits of a slice's projection depend on the stack it is in; the
+    C entry ``gr_radon`` always gathers.
     """
     g = _geom(r_struct)
     nx, ny = g.shape

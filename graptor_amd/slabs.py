@@ -10,8 +10,10 @@ and pbar of the plane below it, its primal step v_z of the plane below and
 Ranks would exchange these planes with their neighbours twice per iteration
 (send / receive pairs over xGMI) as buffers packed by gr_tgv_pack_halos;
 here all slabs share one GPU and each slab packs its planes straight into
-its neighbours' halo fields, so the result equals the unsplit volume's solve
-bit for bit.
+its neighbours' halo fields, so the result equals the same steps on the unsplit
+volume (one slab) bit for bit.  It also equals ``TgvProblem.iterate``'s except
+for the rounding of the KL prox of large stacks, which that fuses into the
+projection.
 
 The iteration is composed from the single-step entry points (dual step,
 forward projection, prox, backprojection, primal step) so that the halo

@@ -50,7 +50,8 @@ int gr_radon_struct(const double *angles, int na, int nx, int ny, int nd,
 
 /* Device-side form of r_struct (2D:531-535): the angle table plus the
  * projector's per-angle constants and work chunks.  ofs is a host table
- * ofs[na][4] as produced by gr_radon_struct. */
+ * ofs[na][4] as produced by gr_radon_struct.  Any detector width; batch plans
+ * and the fused primal step refuse bins of less than about 1/150 pixel. */
 typedef struct gr_geometry gr_geometry;
 int gr_geometry_create(const float *ofs, int na, int nx, int ny, int nd,
                        gr_geometry **out);
@@ -73,10 +74,13 @@ int gr_iterates_by_lines(const gr_geometry *g, int nslices);
 int gr_radon(const gr_geometry *g, float *sino, const float *img, int nslices,
              void *stream);
 /* The same with a scratch array of at least gr_radon_scratch_floats floats, which
- * is overwritten and overlaps neither img nor sino: small stacks are then projected by lines, two
- * to seven times as fast.  0 floats: gr_radon does as well.  of_slices > 0: the
- * slices are part of a stack of so many and get the bits that an iteration of
- * the whole stack gives them (scratch: as large as img). */
+ * is overwritten and overlaps neither img nor sino: small stacks are then
+ * projected by lines, up to seven times as fast for a few large slices and about
+ * as fast where the number of floats turns 0, with which gr_radon does as well.
+ * The two ways round differently, so a slice's last bits depend on the stack it is
+ * in (gr_radon's do not).  of_slices > 0: the slices are part of a stack of so many
+ * and get the bits that an iteration of the whole stack gives them (scratch: as
+ * large as img). */
 size_t gr_radon_scratch_floats(const gr_geometry *g, int nslices);
 int gr_radon_scratch(const gr_geometry *g, float *sino, const float *img, int nslices,
                      float *scratch, int of_slices, void *stream);
