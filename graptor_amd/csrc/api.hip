@@ -373,16 +373,23 @@ struct gr_plan {
     int nprob = 0;
     std::vector<ProbDev> probs;
     ProbDev* probs_dev = nullptr;
-    // mi: items per thread, or 0: by lines, in work-groups of `waves` waves
+    // mi: items per thread, or 0: by lines, in work-groups of `waves` waves (K:
+    // the most slices of an item)
     struct FwdLaunch {
         int K, mi; size_t lds; std::vector<FwdItem> items; FwdItem* dev; int waves = 0;
-        bool wide = false;
+        bool wide = false, mixed = false;  // mixed: gathered items and items by lines
+        bool one_k = true;                 // by lines: every item has K slices
     };
     struct AdjLaunch { int K, dim, tgv, fuse; size_t lds; std::vector<AdjItem> items; AdjItem* dev; };
     struct PrimalLaunch { int dim, tgv; std::vector<DualItem> items; DualItem* dev; };
-    struct DualLaunch { int dim, coupling, tgv, maxc; std::vector<DualItem> items; DualItem* dev; };
+    struct DualLaunch {
+        int dim, coupling, tgv, maxc; std::vector<DualItem> items; DualItem* dev;
+        bool tiles = false;  // transposes for the launch by lines
+    };
     std::vector<FwdLaunch> fwd;
-    std::vector<DualItem> tiles;  // 32 x 32 tiles transposed ahead of the launches by lines
+    // 32 x 32 tiles transposed ahead of the launch by lines, unless a launch of
+    // the dual step holds them
+    std::vector<DualItem> tiles;
     DualItem* tiles_dev = nullptr;
     std::vector<AdjLaunch> adj;
     std::vector<DualLaunch> dual;
@@ -416,6 +423,23 @@ void plan_free_device(gr_plan* pl)
     pl->graph_block = 0;
 }
 
+// Below this many voxel-channels a batch iteration keeps the four phases in
+// sequence: its kernels are latency-bound, and the extra fork and launch of
+// the three-fork order cost more than the overlap gains (183x183, one
+// channel, graph replay: 0.0887 against 0.0821 ms per iteration; 64 2D
+// problems, 11.5 M voxel-channels: 1.033 against 1.108 ms).
+constexpr double PLAN_OVERLAP_MIN = 1 << 20;
+
+// Work-groups of the dual step are those of transpose_tile.
+constexpr bool DUAL_TRANSPOSES = DUAL_BX * DUAL_BY == 256;
+
+bool plan_overlaps(const gr_plan* pl)
+{
+    double vc = 0.0;
+    for (const auto& P : pl->probs) vc += (double)P.nx * P.ny * P.nz * P.nch;
+    return vc >= PLAN_OVERLAP_MIN;
+}
+
 int plan_build(gr_plan* pl, const gr_geometry* const* geoms)
 {
     plan_free_device(pl);
@@ -425,14 +449,25 @@ int plan_build(gr_plan* pl, const gr_geometry* const* geoms)
     pl->dual.clear();
     pl->primal.clear();
     const int n = pl->nprob;
-    // forward chunk tables: a common target of (bin, line) pairs per
-    // work-group (the batch's total over ~3 work-groups per CU); each problem
-    // takes the items-per-thread table whose chunks come closest to it
+    // forward chunk tables of the problems that gather: a common target of
+    // (bin, line) pairs per work-group (their total over ~3 work-groups per
+    // CU; with the total of all problems a plan of 64 slices of 48^2 to 125^2
+    // took 264 us an iteration, so 185); each takes the items-per-thread table
+    // whose chunks come closest to it
+    const bool overlaps = plan_overlaps(pl);
     double total_work = 0.0;
+    int line_waves = overlaps ? FWD_LINE_WAVES : 0;  // per work-group by lines
+    bool short_lines = false;
     for (int i = 0; i < n; ++i) {
         const ProbDev& P = pl->probs[i];
         const int S = P.nz * P.nch, K = slice_group(S);
-        total_work += (double)((S + K - 1) / K) * P.na * P.nd * std::max(P.nx, P.ny);
+        if (fwd_by_lines(P, geoms[i]->g)) {
+            const int J = geoms[i]->g.shear_waves;
+            line_waves = std::max(line_waves, J);
+            short_lines = short_lines || J <= FWD_THREADS / 64;
+        } else {
+            total_work += (double)((S + K - 1) / K) * P.na * P.nd * std::max(P.nx, P.ny);
+        }
     }
     const double target = std::max(1.0, total_work / 768.0);
     std::vector<int> tsel(n, 0);
@@ -451,11 +486,18 @@ int plan_build(gr_plan* pl, const gr_geometry* const* geoms)
         }
         if (g.wide_bins) tsel[i] = FWD_WIDE_TABLE;
     }
-    // waves per work-group of the launches by lines
-    int line_waves = FWD_LINE_WAVES;
+    // Phases in sequence: a launch and its fork cost as much as a small
+    // projection, so all items by lines go into one launch, whatever their K,
+    // and where they are no longer than a gathered item's work-group into one
+    // with these (of one item per thread).  us an iteration, one launch per K
+    // and kind / so: 18 slices of 62^2 to 104^2 160 / 104, of one channel 85 /
+    // 64 (gathered altogether 68); 8 of 80^2 to 120^2 140 / 103.  Beside the
+    // stencil steps of larger plans the launches of a K keep their registers:
+    // 64 of 100^2 to 384^2, one channel, 272 / 284.
+    bool mixed = false;
     for (int i = 0; i < n; ++i)
-        if (fwd_by_lines(pl->probs[i], geoms[i]->g))
-            line_waves = std::max(line_waves, geoms[i]->g.shear_waves);
+        mixed = mixed || (8 >> tsel[i] == 1 && !fwd_by_lines(pl->probs[i], geoms[i]->g));
+    mixed = mixed && DUAL_TRANSPOSES && !overlaps && short_lines;
     std::map<std::tuple<int, int, int>, size_t> fwd_idx;
     std::map<std::tuple<int, int, int, int>, size_t> adj_idx;
     std::map<std::tuple<int, int>, size_t> primal_idx;
@@ -465,39 +507,40 @@ int plan_build(gr_plan* pl, const gr_geometry* const* geoms)
         const Geometry& g = geoms[i]->g;
         const int S = P.nz * P.nch;
         const int K = slice_group(S);
-        if (fwd_by_lines(P, g)) {
-            // slice groups x runs of angles that fill line_waves waves of items
-            const int J = g.shear_waves;
-            auto fk = std::make_tuple(K, 0, 0);
-            if (!fwd_idx.count(fk)) {
-                fwd_idx[fk] = pl->fwd.size();
-                pl->fwd.push_back({K, 0, 0, {}, nullptr});
-                pl->fwd.back().waves = line_waves;
-            }
-            auto& fl = pl->fwd[fwd_idx[fk]];
-            const int per = line_waves / J;
+        const bool by_lines = fwd_by_lines(P, g);
+        const int t = tsel[i];
+        const bool mix = mixed && (by_lines ? g.shear_waves <= FWD_THREADS / 64 : 8 >> t == 1);
+        const int mi = mix ? 1 : by_lines ? 0 : 8 >> t;
+        auto fk = std::make_tuple(mix || (by_lines && !overlaps) ? 0 : K, mi,
+                                  by_lines ? 0 : g.wide_bins);
+        if (!fwd_idx.count(fk)) {
+            fwd_idx[fk] = pl->fwd.size();
+            pl->fwd.push_back({K, mi, 0, {}, nullptr});
+            auto& l = pl->fwd.back();
+            l.waves = mix ? FWD_THREADS / 64 : line_waves;
+            l.wide = !by_lines && g.wide_bins;
+            l.mixed = mix;
+        }
+        auto& fl = pl->fwd[fwd_idx[fk]];
+        fl.one_k = fl.one_k && fl.K == K;
+        fl.K = std::max(fl.K, K);
+        if (by_lines) {
+            // slice groups x runs of angles that fill the waves with items
+            const int J = g.shear_waves, per = fl.waves / J;
             for (int s0 = 0; s0 < S; s0 += K)
                 for (int a = 0; a < P.na; a += per)
-                    fl.items.push_back(FwdItem{i, J, a, std::min(per, P.na - a), 0, 0, s0, 0});
+                    fl.items.push_back(FwdItem{i, J, a, std::min(per, P.na - a), 0, 0, s0, K});
             for (int sl = 0; sl < S; ++sl)
                 for (int y0 = 0; y0 < P.ny; y0 += 32)
                     for (int x0 = 0; x0 < P.nx; x0 += 32)
                         pl->tiles.push_back(DualItem{i, x0, y0, sl});
         } else {
             // slice groups x chunks (group-major)
-            const int t = tsel[i], mi = 8 >> t;
-            auto fk = std::make_tuple(K, mi, g.wide_bins);
-            if (!fwd_idx.count(fk)) {
-                fwd_idx[fk] = pl->fwd.size();
-                pl->fwd.push_back({K, mi, 0, {}, nullptr});
-                pl->fwd.back().wide = g.wide_bins != 0;
-            }
-            auto& fl = pl->fwd[fwd_idx[fk]];
             fl.lds = std::max(fl.lds, fwd_lds_bytes(P, K));
             for (int s0 = 0; s0 < S; s0 += K)
                 for (int c = g.tab_off[t]; c < g.tab_off[t + 1]; ++c) {
                     const FwdChunk& ch = g.chunks_host[c];
-                    fl.items.push_back(FwdItem{i, ch.cls, ch.a0, ch.na, ch.b0, ch.nb, s0, 0});
+                    fl.items.push_back(FwdItem{i, ch.cls, ch.a0, ch.na, ch.b0, ch.nb, s0, K});
                 }
         }
         // backprojection + primal items: tiles x slice groups
@@ -541,11 +584,38 @@ int plan_build(gr_plan* pl, const gr_geometry* const* geoms)
             for (int y0 = 0; y0 < P.ny; y0 += DUAL_BY)
                 for (int x0 = 0; x0 < P.nx; x0 += DUAL_BX) dl.items.push_back(DualItem{i, x0, y0, z});
     }
+    // phases in sequence: the dual step, which comes first and does not touch
+    // K^T lambda, transposes beside its own tiles (a launch of its own: 5 us)
+    if (DUAL_TRANSPOSES && !overlaps && !pl->tiles.empty()) {
+        auto& l = pl->dual[0];
+        for (DualItem t : pl->tiles) {
+            t.prob = ~t.prob;
+            l.items.push_back(t);
+        }
+        l.tiles = true;
+        pl->tiles.clear();
+    }
     // largest chunks first, so the smallest fill the tail of the launch
     for (auto& l : pl->fwd) {
-        if (l.mi == 0) continue;  // of about one size, in the order of the images
+        if (l.mi == 0) {
+            // in the order of the images; of several K, each XCD takes an eighth
+            // of each, the largest first (21 slices of 109^2 to 117^2: 155 us an
+            // iteration as they come, 148 so)
+            std::vector<FwdItem> dealt;
+            for (int x = 0; x < 8 && !l.one_k; ++x)
+                for (int k = 4; k > 0; k /= 2) {
+                    std::vector<FwdItem> of_k;
+                    for (const FwdItem& it : l.items)
+                        if (it.k == k) of_k.push_back(it);
+                    dealt.insert(dealt.end(), of_k.begin() + of_k.size() * x / 8,
+                                 of_k.begin() + of_k.size() * (x + 1) / 8);
+                }
+            if (!l.one_k) l.items.swap(dealt);
+            continue;
+        }
         auto work = [&](const FwdItem& it) {
             const ProbDev& P = pl->probs[it.prob];
+            if (it.nb == 0) return 1e30;  // by lines: whole lines in a wave
             return (double)it.na * it.nb * (it.cls == 0 ? P.nx : P.ny);
         };
         std::stable_sort(l.items.begin(), l.items.end(),
@@ -666,12 +736,15 @@ int plan_phase(gr_plan* pl, int phase, int fwd_mode, hipStream_t st)
         if (ph == 0) {
             const auto& l = pl->dual[i];
             rc = launch_dual_batch(pl->probs_dev, l.dev, (int)l.items.size(), l.dim, l.coupling,
-                                   l.tgv != 0, l.maxc, s);
+                                   l.tgv != 0, l.maxc, l.tiles, s);
         } else if (ph == 1) {
             const auto& l = pl->fwd[i];
             if (l.mi == 0)
                 rc = launch_fwd_line_batch(pl->probs_dev, l.dev, (int)l.items.size(), l.K,
-                                           l.waves, fwd_mode, s);
+                                           l.one_k, l.waves, fwd_mode, s);
+            else if (l.mixed)
+                rc = launch_fwd_mixed_batch(pl->probs_dev, l.dev, (int)l.items.size(), l.K,
+                                            l.lds, fwd_mode, s);
             else
                 rc = launch_fwd_batch(pl->probs_dev, l.dev, (int)l.items.size(), l.K, l.mi,
                                       l.wide, l.lds, fwd_mode, s);
@@ -694,18 +767,9 @@ int plan_phase(gr_plan* pl, int phase, int fwd_mode, hipStream_t st)
     return rc;
 }
 
-// Below this many voxel-channels a batch iteration keeps the four phases in
-// sequence: its kernels are latency-bound, and the extra fork and launch of
-// the three-fork order cost more than the overlap gains (183x183, one
-// channel, graph replay: 0.0887 against 0.0821 ms per iteration; 64 2D
-// problems, 11.5 M voxel-channels: 1.033 against 1.108 ms).
-constexpr double PLAN_OVERLAP_MIN = 1 << 20;
-
 int plan_iter(gr_plan* pl, int n_iter, int ku_on_last, hipStream_t st)
 {
-    double vc = 0.0;
-    for (const auto& P : pl->probs) vc += (double)P.nx * P.ny * P.nz * P.nch;
-    const bool overlap = vc >= PLAN_OVERLAP_MIN;
+    const bool overlap = plan_overlaps(pl);
     for (int it = 0; it < n_iter; ++it) {
         const int mode = FWD_PROX | ((ku_on_last && it == n_iter - 1) ? FWD_WRITE : 0);
         int rc = GR_OK;

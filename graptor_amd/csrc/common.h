@@ -102,10 +102,11 @@ struct FusedBufs {
     float *u_out, *p_out, *v_out, *w_out;
 };
 
-struct FwdItem { int prob, cls, a0, na, b0, nb, s0, pad; };
+struct FwdItem { int prob, cls, a0, na, b0, nb, s0, k; };
 struct AdjItem { int prob, x0, y0, s0; };
 // Stencil items: a 64 x 4 tile of plane z (dual step) or of slice
-// z + nz * channel (primal step).
+// z + nz * channel (primal step).  prob < 0 among dual items: a 32 x 32 tile of
+// slice z of problem ~prob, transposed for the projection by lines.
 struct DualItem { int prob, x0, y0, z; };
 
 // Chunk table (FWD_THREADS x 8 >> t items) of geometries with wide bins, the only
@@ -253,6 +254,28 @@ __device__ __forceinline__ int stencil_block()
     return ((local / G) * 8 + xcd) * G + local % G;
 }
 
+// P.ktl = slice s of P.ubar transposed, one 32 x 32 tile, by 256 threads
+// through TRANSPOSE_FLOATS floats of LDS.
+constexpr int TRANSPOSE_FLOATS = 32 * 33;
+__device__ __forceinline__ void transpose_tile(float* tile, const ProbDev& P, int s, int x0,
+                                               int y0)
+{
+    const int nx = P.nx, ny = P.ny, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    const float* __restrict__ src = P.ubar + (size_t)s * nx * ny;
+    float* __restrict__ dst = P.ktl + (size_t)s * nx * ny;
+#pragma unroll
+    for (int r = 0; r < 32; r += 8) {
+        const int x = x0 + tx, y = y0 + ty + r;
+        if (x < nx && y < ny) tile[(ty + r) * 33 + tx] = src[(size_t)y * nx + x];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 32; r += 8) {
+        const int x = x0 + ty + r, y = y0 + tx;
+        if (x < nx && y < ny) dst[(size_t)x * ny + y] = tile[tx * 33 + ty + r];
+    }
+}
+
 inline void set_shear(ProbDev& P, const Geometry& g)
 {
     P.shear = g.shear_dev; P.lines = g.lines_dev; P.line0 = g.line0_dev; P.bins = g.bins_dev;
@@ -300,18 +323,26 @@ int launch_primal_part(const ProbDev& P, int part, hipStream_t st);
 int launch_fwd_batch(const ProbDev* probs_dev, const FwdItem* items, int nitems, int K,
                      int mi, bool wide, size_t lds, int mode, hipStream_t st);
 // The sheared forward projection of batch problems: items {prob, J, first
-// angle, angles, 0, 0, s0} of K slices, J = waves of items of one angle and
-// angles * J <= waves; after launch_transpose_batch (items: 32 x 32 tiles x0,
-// y0 of slice z).  With FWD_LINE_WAVES waves the forward phase of 64 mixed
-// slices (96^2 to 384^2) takes 0.45 ms; with 9, 10 and 16: 0.58, 0.56, 0.54
-// (a multiple of 4 loads the SIMDs evenly, and 16 leave room for one
-// work-group less); one launch per J 0.48.
+// angle, angles, 0, 0, s0, slices} of at most K slices, J = waves of items of
+// one angle and angles * J <= waves; the slices are transposed before, by
+// launch_transpose_batch (items: 32 x 32 tiles x0, y0 of slice z) or the dual
+// step.  With FWD_LINE_WAVES waves the forward phase of 64 mixed slices (96^2
+// to 384^2) takes 0.45 ms; with 9, 10 and 16: 0.58, 0.56, 0.54 (a multiple of 4
+// loads the SIMDs evenly, and 16 leave room for one work-group less); one
+// launch per J 0.48.  Small plans have work-groups of one angle: 28 slices of
+// 89^2 to 130^2 117 us an iteration, 130 with 12 waves.  one_k: every item has
+// K slices.
 constexpr int FWD_LINE_WAVES = 12;
 int launch_fwd_line_batch(const ProbDev* probs_dev, const FwdItem* items, int nitems, int K,
-                          int waves, int mode, hipStream_t st);
+                          bool one_k, int waves, int mode, hipStream_t st);
 // Fills the tables of the sheared projection (line0 is there; first: each angle's
 // first item) and waits.
 int launch_line_tables(const Geometry& g, const int* first);
+// Gathered items (FWD_THREADS chunks of one item per thread, unit bins) and items
+// by lines (nb = 0, FWD_THREADS / 64 waves) of at most K slices, in one launch;
+// lds: bytes that the former need.
+int launch_fwd_mixed_batch(const ProbDev* probs_dev, const FwdItem* items, int nitems, int K,
+                           size_t lds, int mode, hipStream_t st);
 int launch_transpose_batch(const ProbDev* probs_dev, const DualItem* items, int nitems,
                            hipStream_t st);
 // Whether an iteration of this problem (alone: a projection outside one)
@@ -322,7 +353,7 @@ int launch_adj_batch(const ProbDev* probs_dev, const AdjItem* items, int nitems,
 int launch_primal_batch(const ProbDev* probs_dev, const DualItem* items, int nitems, int dim,
                         bool tgv, int part, hipStream_t st);
 int launch_dual_batch(const ProbDev* probs_dev, const DualItem* items, int nitems, int dim,
-                      int coupling, bool tgv, int maxc, hipStream_t st);
+                      int coupling, bool tgv, int maxc, bool tiles, hipStream_t st);
 
 // ---- auxiliary (aux.hip) ---------------------------------------------------
 int launch_normest(const Geometry& g, const double* x0_host, int iters, int mode,

@@ -243,6 +243,22 @@ __global__ __launch_bounds__(1024) void fwd_line_kernel(ProbDev P, int J, int ns
     fwd_line_body<K>(P, work % P.na, 1, (work / P.na) * K, J, ns, mode, sh);
 }
 
+// An item by lines of a batch, of K slices, or (K = 0) as many as it says.
+template <int K>
+__device__ __forceinline__ void fwd_line_item(const ProbDev& P, const FwdItem& I, int mode,
+                                              float* sh)
+{
+    if constexpr (K > 0) {
+        fwd_line_body<K>(P, I.a0, I.na, I.s0, I.cls, 1, mode, sh);
+    } else {
+        switch (I.k) {
+        case 4: fwd_line_body<4>(P, I.a0, I.na, I.s0, I.cls, 1, mode, sh); break;
+        case 2: fwd_line_body<2>(P, I.a0, I.na, I.s0, I.cls, 1, mode, sh); break;
+        default: fwd_line_body<1>(P, I.a0, I.na, I.s0, I.cls, 1, mode, sh);
+        }
+    }
+}
+
 template <int K>
 __global__ __launch_bounds__(1024) void fwd_line_batch_kernel(const ProbDev* __restrict__ probs,
                                                               const FwdItem* __restrict__ items,
@@ -250,8 +266,7 @@ __global__ __launch_bounds__(1024) void fwd_line_batch_kernel(const ProbDev* __r
 {
     extern __shared__ float sh[];
     const FwdItem I = items[xcd_work_id(blockIdx.x, gridDim.x)];
-    const ProbDev P = load_prob(probs, I.prob);
-    fwd_line_body<K>(P, I.a0, I.na, I.s0, I.cls, 1, mode, sh);
+    fwd_line_item<K>(load_prob(probs, I.prob), I, mode, sh);
 }
 
 // Tables of the sheared projection, a work-group per angle.  In 64 bits the
@@ -298,38 +313,20 @@ __global__ __launch_bounds__(256) void line_tables_kernel(const FwdAngle* __rest
     }
 }
 
-// P.ktl = slice s of P.ubar transposed, one 32 x 32 tile through LDS.
-__device__ __forceinline__ void transpose_tile(const ProbDev& P, int s, int x0, int y0)
-{
-    __shared__ float tile[32][33];
-    const int nx = P.nx, ny = P.ny, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-    const float* __restrict__ src = P.ubar + (size_t)s * nx * ny;
-    float* __restrict__ dst = P.ktl + (size_t)s * nx * ny;
-#pragma unroll
-    for (int r = 0; r < 32; r += 8) {
-        const int x = x0 + tx, y = y0 + ty + r;
-        if (x < nx && y < ny) tile[ty + r][tx] = src[(size_t)y * nx + x];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < 32; r += 8) {
-        const int x = x0 + ty + r, y = y0 + tx;
-        if (x < nx && y < ny) dst[(size_t)x * ny + y] = tile[tx][ty + r];
-    }
-}
-
 __global__ __launch_bounds__(256) void transpose_kernel(ProbDev P, int tiles_x, int tiles_y)
 {
+    __shared__ float tile[TRANSPOSE_FLOATS];
     const int tiles = tiles_x * tiles_y, t = blockIdx.x % tiles;
-    transpose_tile(P, blockIdx.x / tiles, 32 * (t % tiles_x), 32 * (t / tiles_x));
+    transpose_tile(tile, P, blockIdx.x / tiles, 32 * (t % tiles_x), 32 * (t / tiles_x));
 }
 
 __global__ __launch_bounds__(256) void transpose_batch_kernel(const ProbDev* __restrict__ probs,
                                                               const DualItem* __restrict__ items)
 {
+    __shared__ float tile[TRANSPOSE_FLOATS];
     const DualItem I = items[blockIdx.x];
     const ProbDev P = load_prob(probs, I.prob);
-    transpose_tile(P, I.z, I.x0, I.y0);
+    transpose_tile(tile, P, I.z, I.x0, I.y0);
 }
 
 // --------------------------------------------------------------------------
@@ -536,6 +533,25 @@ __global__ __launch_bounds__(FWD_THREADS) void fwd_batch_kernel(const ProbDev* _
     const FwdItem I = items[blockIdx.x];
     const ProbDev P = load_prob(probs, I.prob);
     fwd_body<K, MI, WIDE>(P, I, mode, sh);
+}
+
+// A small batch's gathered items and its items by lines: bound by the latency of
+// one work-group and by the launch, of which two need two.
+__global__ __launch_bounds__(FWD_THREADS) void fwd_mixed_batch_kernel(
+    const ProbDev* __restrict__ probs, const FwdItem* __restrict__ items, int mode)
+{
+    extern __shared__ float sh[];
+    const FwdItem I = items[blockIdx.x];
+    const ProbDev P = load_prob(probs, I.prob);
+    if (I.nb == 0) {
+        fwd_line_item<0>(P, I, mode, sh);
+        return;
+    }
+    switch (I.k) {
+    case 4: fwd_body<4, 1, false>(P, I, mode, sh); break;
+    case 2: fwd_body<2, 1, false>(P, I, mode, sh); break;
+    default: fwd_body<1, 1, false>(P, I, mode, sh);
+    }
 }
 
 // --------------------------------------------------------------------------
@@ -1368,6 +1384,16 @@ int launch_line_tables(const Geometry& g, const int* first)
     return GR_OK;
 }
 
+int launch_fwd_mixed_batch(const ProbDev* probs, const FwdItem* items, int nitems, int K,
+                           size_t lds, int mode, hipStream_t st)
+{
+    if (nitems <= 0) return GR_OK;
+    hipLaunchKernelGGL(fwd_mixed_batch_kernel, dim3((unsigned)nitems), dim3(FWD_THREADS),
+                       std::max(lds, fwd_line_lds(K, FWD_THREADS / 64)), st, probs, items, mode);
+    GR_LAUNCH_CHECK("fwd_mixed_batch_kernel");
+    return GR_OK;
+}
+
 int launch_transpose_batch(const ProbDev* probs, const DualItem* items, int nitems,
                            hipStream_t st)
 {
@@ -1379,17 +1405,18 @@ int launch_transpose_batch(const ProbDev* probs, const DualItem* items, int nite
 }
 
 int launch_fwd_line_batch(const ProbDev* probs, const FwdItem* items, int nitems, int K,
-                          int waves, int mode, hipStream_t st)
+                          bool one_k, int waves, int mode, hipStream_t st)
 {
     if (nitems <= 0) return GR_OK;
     const dim3 grd((unsigned)nitems), blk(64 * waves);
     const size_t lds = fwd_line_lds(K, waves);
-    if (K == 4)
-        hipLaunchKernelGGL((fwd_line_batch_kernel<4>), grd, blk, lds, st, probs, items, mode);
-    else if (K == 2)
-        hipLaunchKernelGGL((fwd_line_batch_kernel<2>), grd, blk, lds, st, probs, items, mode);
-    else
-        hipLaunchKernelGGL((fwd_line_batch_kernel<1>), grd, blk, lds, st, probs, items, mode);
+#define GR_FL(KK) \
+    hipLaunchKernelGGL(fwd_line_batch_kernel<KK>, grd, blk, lds, st, probs, items, mode)
+    if (!one_k) GR_FL(0);
+    else if (K == 4) GR_FL(4);
+    else if (K == 2) GR_FL(2);
+    else GR_FL(1);
+#undef GR_FL
     GR_LAUNCH_CHECK("fwd_line_batch_kernel");
     return GR_OK;
 }

@@ -502,7 +502,12 @@ template <int DIM, int CPL, bool TGV, int MAXC>
 __global__ __launch_bounds__(DUAL_BX* DUAL_BY) void dual_batch_kernel(
     const ProbDev* __restrict__ probs, const DualItem* __restrict__ items)
 {
+    extern __shared__ float sh[];
     const DualItem I = items[blockIdx.x];
+    if (I.prob < 0) {
+        transpose_tile(sh, load_prob(probs, ~I.prob), I.z, I.x0, I.y0);
+        return;
+    }
     const ProbDev P = load_prob(probs, I.prob);
     dual_body<DIM, CPL, TGV, MAXC>(P, I);
 }
@@ -522,7 +527,12 @@ template <int DIM, int CPL, bool TGV>
 __global__ __launch_bounds__(DUAL_BX* DUAL_BY) void dual_wide_batch_kernel(
     const ProbDev* __restrict__ probs, const DualItem* __restrict__ items)
 {
+    extern __shared__ float sh[];
     const DualItem I = items[blockIdx.x];
+    if (I.prob < 0) {
+        transpose_tile(sh, load_prob(probs, ~I.prob), I.z, I.x0, I.y0);
+        return;
+    }
     const ProbDev P = load_prob(probs, I.prob);
     dual_body_wide<DIM, CPL, TGV>(P, I);
 }
@@ -1039,17 +1049,18 @@ int launch_dual(const ProbDev& P, hipStream_t st)
 }
 
 int launch_dual_batch(const ProbDev* probs, const DualItem* items, int nitems, int dim,
-                      int coupling, bool tgv, int maxc, hipStream_t st)
+                      int coupling, bool tgv, int maxc, bool tiles, hipStream_t st)
 {
     if (nitems <= 0) return GR_OK;
+    const size_t lds = tiles ? TRANSPOSE_FLOATS * sizeof(float) : 0;
     dim3 grd((unsigned)nitems), blk(DUAL_BX * DUAL_BY);
 #define GR_DB(DD, CC, TT, MM) \
-    hipLaunchKernelGGL((dual_batch_kernel<DD, CC, TT, MM>), grd, blk, 0, st, probs, items)
+    hipLaunchKernelGGL((dual_batch_kernel<DD, CC, TT, MM>), grd, blk, lds, st, probs, items)
 #define GR_DB_M(DD, CC, TT)                                                                 \
     do {                                                                                    \
         if (maxc <= 4) GR_DB(DD, CC, TT, 4);                                                \
         else if (maxc <= 8) GR_DB(DD, CC, TT, 8);                                           \
-        else hipLaunchKernelGGL((dual_wide_batch_kernel<DD, CC, TT>), grd, blk, 0, st, probs, \
+        else hipLaunchKernelGGL((dual_wide_batch_kernel<DD, CC, TT>), grd, blk, lds, st, probs, \
                                 items);                                                     \
     } while (0)
 #define GR_DB_T(DD, CC) \
