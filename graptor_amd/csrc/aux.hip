@@ -222,8 +222,9 @@ int launch_normest(const Geometry& g, const double* x0_host, int iters, int mode
     if (rc == GR_OK) image(nullptr, nullptr);
     double result = 0.0, prev = 0.0, h[2] = {0.0, 0.0};  // norm, dot
     for (int it = 0; it < iters && rc == GR_OK; ++it) {
-        hipLaunchKernelGGL(g.wide_bins ? fwd64_kernel<true> : fwd64_kernel<false>, dim3(fb), dim3(T64), 0, st, x, xt, s, g.fwd_dev, g.nx,
-                           g.ny, g.nd, parts, np, power ? 1 : 0, red);
+        hipLaunchKernelGGL(g.wide_bins ? fwd64_kernel<true> : fwd64_kernel<false>, dim3(fb),
+                           dim3(T64), 0, st, x, xt, s, g.fwd_dev, g.nx, g.ny, g.nd, parts, np,
+                           power ? 1 : 0, red);
         image(s, power ? dots : nullptr);
         chk(hipGetLastError(), "normest launch");
         if (!power && it + 1 < iters) continue;
