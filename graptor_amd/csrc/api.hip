@@ -440,14 +440,8 @@ bool plan_overlaps(const gr_plan* pl)
     return vc >= PLAN_OVERLAP_MIN;
 }
 
-int plan_build(gr_plan* pl, const gr_geometry* const* geoms)
+int plan_fill(gr_plan* pl, const gr_geometry* const* geoms)
 {
-    plan_free_device(pl);
-    pl->fwd.clear();
-    pl->tiles.clear();
-    pl->adj.clear();
-    pl->dual.clear();
-    pl->primal.clear();
     const int n = pl->nprob;
     // forward chunk tables of the problems that gather: a common target of
     // (bin, line) pairs per work-group (their total over ~3 work-groups per
@@ -633,6 +627,31 @@ int plan_build(gr_plan* pl, const gr_geometry* const* geoms)
     for (auto& l : pl->dual) if (!rc) rc = upload(l.items, &l.dev);
     for (auto& l : pl->primal) if (!rc) rc = upload(l.items, &l.dev);
     return rc;
+}
+
+void plan_clear(gr_plan* pl)
+{
+    plan_free_device(pl);
+    pl->fwd.clear();
+    pl->tiles.clear();
+    pl->adj.clear();
+    pl->dual.clear();
+    pl->primal.clear();
+}
+
+// A plan that could not be built has no tables and no launches.
+int plan_build(gr_plan* pl, const gr_geometry* const* geoms)
+{
+    plan_clear(pl);
+    const int rc = plan_fill(pl, geoms);
+    if (rc) plan_clear(pl);
+    return rc;
+}
+
+bool plan_built(const gr_plan* pl)
+{
+    if (!pl->probs_dev) set_error("plan: its last retune failed");
+    return pl->probs_dev != nullptr;
 }
 
 int plan_lanes(gr_plan* pl)
@@ -1253,6 +1272,7 @@ int gr_plan_iterate(gr_plan* pl, int n_iter, int ku_on_last, void* stream)
         set_error("plan_iterate: invalid arguments");
         return GR_ERR_INVALID;
     }
+    if (!plan_built(pl)) return GR_ERR_INVALID;
     if (ku_on_last)
         for (const auto& P : pl->probs)
             if (!P.ku) {
@@ -1268,6 +1288,7 @@ int gr_plan_iterate_graph(gr_plan* pl, int n_iter, int block, void* stream)
         set_error("plan_iterate_graph: invalid arguments");
         return GR_ERR_INVALID;
     }
+    if (!plan_built(pl)) return GR_ERR_INVALID;
     hipStream_t st = stream_of(stream);
     {
         // the graph is captured on a private stream and replayed on `stream`;
@@ -1317,6 +1338,7 @@ int gr_plan_profile(gr_plan* pl, int n_iter, double* ms_out, void* stream)
         set_error("plan_profile: invalid arguments");
         return GR_ERR_INVALID;
     }
+    if (!plan_built(pl)) return GR_ERR_INVALID;
     hipStream_t st = stream_of(stream);
     hipEvent_t ev[5];
     for (int k = 0; k < 5; ++k) GR_HIP(hipEventCreate(&ev[k]));

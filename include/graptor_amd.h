@@ -247,7 +247,9 @@ int gr_plan_iterate_graph(gr_plan *plan, int n_iter, int block, void *stream);
  * iterations.  Synchronises the stream. */
 int gr_plan_profile(gr_plan *plan, int n_iter, double *ms_out, void *stream);
 /* Re-reads every geometry's tile shapes (gr_geometry_set_tuning) into the
- * plan; used by the tile autotuner.  Drops a captured graph. */
+ * plan; used by the tile autotuner.  Drops a captured graph.  After a failure
+ * (shapes that do not fit LDS) the plan refuses to iterate until a retune
+ * succeeds. */
 int gr_plan_retune(gr_plan *plan, const gr_geometry *const *geoms);
 
 /* ------------------------------------------------------------------------
