@@ -24,6 +24,8 @@ PLANS = {
     "lines of more waves and gather": [(60, 20, 1, "TGV", 1.0), (260, 40, 2, "TGV", 1.0)],
     "lines, one slice": [(90, 20, 1, "TGV", 1.0), (120, 17, 1, "TGV", 1.0)],
     "lines, groups of 2 and 4": [(90, 20, 2, "TGV", 1.0), (120, 17, 4, "TGV", 1.0)],
+    "six channels": [(85, 17, 6, "TGV", 1.0), (60, 20, 1, "TGV", 1.0)],
+    "nine channels": [(85, 17, 9, "TGV", 1.0), (60, 20, 1, "TGV", 1.0)],
     # more than 2^20 voxel-channels: projections beside the stencil steps
     "overlapped": [(64, 20, 1, "TGV", 1.0), (97, 23, 2, "TGV", 1.0), (560, 60, 4, "TGV", 1.0)],
 }
